@@ -21,7 +21,7 @@ LIBRARY = PACKAGE / "liblightdelta_hip.so"
 # torch.ops.lightdelta dispatcher kernels (host C++ over the C ABI; see csrc/torch_ops.cpp)
 TORCH_LIBRARY = PACKAGE / "liblightdelta_torch.so"
 SOURCES = ("abi.hip", "gdn_decode.hip", "prefill_serial.hip", "prefill_chunked.hip",
-           "state_io.hip")
+           "prefill_heads.hip", "state_io.hip")
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [

@@ -15,6 +15,7 @@ constexpr int kPieces = 16;        // 16-byte pieces of the tile per lane
 constexpr int kMaxTokens = LD_MAX_TOKENS;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct DecodeParams {
   const uint16_t* qkv;
@@ -82,8 +83,6 @@ __device__ __forceinline__ f32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, Pol));
 }
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 template <int Pol>
 __device__ __forceinline__ void buffer_store16(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t offset) {
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, offset, 0, Pol);
@@ -139,10 +138,32 @@ inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
   return 32;
 }
 
+// Workspace record of one (32-token chunk, v-head) for chunk_heads_kernel, offsets in bytes:
+// T = (I + A)^-1 diag(beta) and P = P0 T (32 x 32 fp32) as their exact bf16 planes in operand
+// order, plane i of step u at (3 u + i) * 1024 + lane * 16: lane (hi, lj) holds row lj, tokens
+// 16 u + 8 (e / 4) + 4 hi + e % 4, e < 8; then the per-token scales in fp32 (offsets of kSq, ..
+// in 16-byte pieces from kScales) sq = rq scale exp(G), ck = rk exp(G_n-1 - G), ws = rk exp(G),
+// and exp(G_n-1).
+struct HeadRecord {
+  static constexpr int kTokens = 32;
+  static constexpr int kT = 0;
+  static constexpr int kP = 6144;
+  static constexpr int kScales = 12288;
+  static constexpr int kSq = 0;
+  static constexpr int kCk = 8;
+  static constexpr int kWs = 16;
+  static constexpr int kGamma = kScales + 384;
+  static constexpr int kBytes = 12800;
+};
+
 int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequences,
                                         int64_t num_v_heads);
 // chunk_tokens: 64 or 32
+// *normed: whether `out` holds the final outputs (else the raw ones)
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
-                           bool dt_bf16, int chunk_tokens, void* workspace, hipStream_t stream);
+                           bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
+                           hipStream_t stream, bool* normed);
+int launch_chunk_heads(const DecodeParams& p, int num_sequences, const float* ws,
+                       const int32_t* chunk_start, int records, bool w_bf16, hipStream_t stream);
 
 }  // namespace ld

@@ -28,7 +28,9 @@
 //                      point before the gated RMSNorm, which prefill_norm_kernel applies
 //                      afterwards) and the state update.  Rows evolve independently, so a
 //                      head's 128 rows spread over 8 or 4 workgroups.
-//   chunk_scan32_kernel  the same for 32-token chunks, 32 state rows per workgroup.
+//   chunk_scan32_kernel  the same for 32-token chunks, 32 state rows per workgroup; with
+//                      enough (sequence, head) pairs chunk_heads_kernel (prefill_heads.hip)
+//                      instead, a whole head per workgroup with the norm fused.
 // A 64-token chunk costs the same whether it holds 64 tokens or 20, so prompts shorter than
 // a chunk waste the difference; 32-token chunks halve that waste (and the scan's products
 // per token: P V_new grows with the square of the chunk), at twice the sequential steps.
@@ -38,7 +40,7 @@
 // sum over kk of A[i][kk] B[kk][j] to D[i][j], held as d[r] = D[4 lg + r][li].  Summation
 // indices are assigned to (step, lg) freely as long as both operands agree; in the forward
 // substitution k = 4 lg + step, so a result's d[r] is directly the b operand of step r.
-#include "gdn_common.h"
+#include "chunk_common.h"
 
 namespace ld {
 namespace {
@@ -95,9 +97,6 @@ struct Rec32 {
 };
 constexpr int64_t kMiscBeta = 160;
 constexpr int64_t kMiscWs = 192;
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -198,7 +197,6 @@ constexpr int kPrepWaves = kPrepThreads / 64;
 constexpr int kPrepTokens = kC / kPrepWaves;   // tokens normalised per wave
 
 // ---- phase 1: per (chunk, k-head), then per v-head of its group -----------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16v4 __attribute__((ext_vector_type(4)));
 
 // One workgroup per (chunk, k-head).  What depends on q and k alone -- their loads, inverse
@@ -689,6 +687,16 @@ __device__ __forceinline__ int piece32(int mt, int nt, int lg, int li) {
   return ((mt * 2 + (lg & 1)) * 64 + (2 * nt + (lg >> 1)) * 16 + li) * 4;
 }
 
+// Columns j .. j + 3 (j a multiple of 4) of row i of a 32 x 32 matrix into its planes in a
+// HeadRecord (byte offset `base`).
+__device__ __forceinline__ void put_planes(float* rec, int base, int i, int j, f32x4 x) {
+  const Split4 sp = split4(x);
+  uint8_t* at = reinterpret_cast<uint8_t*>(rec) + base + (j >> 4) * 3072 +
+                (((j >> 2) & 1) * 32 + i) * 16 + ((j >> 3) & 1) * 8;
+#pragma unroll
+  for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint2*>(at + pl * 1024) = sp.p[pl];
+}
+
 // The 6 tiles of A (K K^T) and P (Q K^T) on or below the diagonal, as tile_code: A00, A10,
 // A11, P00, P10, P11; wave w takes tiles w and w + 4.
 __device__ __forceinline__ uint32_t prep32_tile(int index) {
@@ -702,13 +710,14 @@ __device__ __forceinline__ uint32_t prep32_tile(int index) {
   }
 }
 
-template <bool DtBf16, bool Wide>
+template <bool DtBf16, bool Wide, bool Heads>
 __global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
 void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
                          const int32_t* chunk_start, int records) {
   using R = Rec32;
   constexpr int kCs = R::kC;
   constexpr int kTokens = kCs / (kPrep32Threads / 64);   // tokens normalised per wave
+  constexpr int64_t kRec = Heads ? HeadRecord::kBytes / 4 : R::kSize;   // floats
   const int64_t unit = blockIdx.x;   // chunk * H + k-head
   const int g = static_cast<int>(unit / p.num_k_heads);
   if (g >= records) return;
@@ -730,9 +739,12 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
   __shared__ __attribute__((aligned(16))) uint16_t sKh[kCs][kHRow];
   __shared__ __attribute__((aligned(16))) float sA[kCs][kARow];     // -A of the v-head
   __shared__ __attribute__((aligned(16))) float sT[3][16][kTRow];   // T0, T1, T10
+  // Heads: P0 of the v-head, double-buffered (the next v-head's is written while waves still
+  // multiply this one's)
+  __shared__ __attribute__((aligned(16))) float sP[Heads ? 2 : 1][Heads ? kCs : 1][kARow];
   // a v-head's gates, double-buffered (v-head m in buffer m & 1): G_i, beta_i, exp(G_i),
   // exp(G_n-1 - G_i), one entry per lane of the wave that forms them
-  __shared__ float sGates[2][4][64];
+  __shared__ __attribute__((aligned(16))) float sGates[2][4][64];
   __shared__ float sRq[kCs];   // rq_i scale (zero past the end)
   __shared__ float sRk[kCs];   // rk_i (zero past the end)
 
@@ -767,7 +779,8 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
     gb[2][lane] = __expf(G);
     gb[3][lane] = __expf(glast - G);
     if (lane == 0)
-      ws[(static_cast<int64_t>(g) * p.num_v_heads + head) * R::kSize + R::kOffMisc] = __expf(glast);
+      ws[(static_cast<int64_t>(g) * p.num_v_heads + head) * kRec +
+         (Heads ? HeadRecord::kGamma / 4 : R::kOffMisc)] = __expf(glast);
   };
   if (wave == 3) fetch_gates(key_head * p.group);
 
@@ -847,7 +860,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
 
   // Qr, Kq and Kr (the bf16 inputs in the scan's load order, item = one 16-byte piece) to
   // the record of the group's first v-head
-  {
+  if constexpr (!Heads) {
     float* rec0 = ws + (static_cast<int64_t>(g) * p.num_v_heads + key_head * p.group) * R::kSize;
     u32x4* qdst = reinterpret_cast<u32x4*>(rec0 + R::kOffQr);
     u32x4* kqdst = reinterpret_cast<u32x4*>(rec0 + R::kOffKq);
@@ -897,7 +910,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
   for (int member = 0; member < p.group; ++member) {
     const int head = key_head * p.group + member;
     const bool next = member + 1 < p.group;
-    float* rec = ws + (static_cast<int64_t>(g) * p.num_v_heads + head) * R::kSize;
+    float* rec = ws + (static_cast<int64_t>(g) * p.num_v_heads + head) * kRec;
     const float* const sG = sGates[member & 1][0];
     const float* const sBeta = sGates[member & 1][1];
     const float* const sEg = sGates[member & 1][2];
@@ -905,7 +918,16 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
 
     // the per-token scales: sq = rq scale exp(G), beta, ck = rk exp(G_n-1 - G),
     // ws = beta exp(G) rk (the 64-token prep's W scale)
-    if (tid < kCs) {
+    if constexpr (Heads) {   // without beta, which is in T's columns
+      constexpr int kAt = HeadRecord::kScales / 4;
+      if (tid < kCs) {
+        rec[kAt + 4 * HeadRecord::kSq + tid] = sRq[tid] * sEg[tid];
+        rec[kAt + 4 * HeadRecord::kWs + tid] = sEg[tid] * sRk[tid];
+      } else if (tid < 2 * kCs) {
+        const int j = tid - kCs;
+        rec[kAt + 4 * HeadRecord::kCk + j] = sRk[j] * sEk[j];
+      }
+    } else if (tid < kCs) {
       rec[R::kOffMisc + kMiscSq + tid] = sRq[tid] * sEg[tid];
       rec[R::kOffMisc + kMiscBeta + tid] = sBeta[tid];
     } else if (tid < 2 * kCs) {
@@ -934,7 +956,10 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
           const float gam = __expf(gi - sG[m]);
           piece[r] = (m <= i && i < len) ? gam * ((rqi * sRk[m]) * prod[t][r]) : 0.0f;
         }
-        *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(mt, nt, lg, li)) = piece;
+        if constexpr (Heads)
+          *reinterpret_cast<f32x4*>(&sP[member & 1][i][16 * nt + 4 * lg]) = piece;
+        else
+          *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(mt, nt, lg, li)) = piece;
       } else {
         const int m = 16 * nt + li;
         const float gm = sG[m];
@@ -947,9 +972,11 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
         }
       }
     }
-    if (wave == 2)
-      *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(0, 1, lg, li)) =
-          f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (!Heads) {
+      if (wave == 2)
+        *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(0, 1, lg, li)) =
+            f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     __syncthreads();   // -A complete
     if (wave == 3 && next) gates(member + 1);
     // inverses of the unit lower-triangular diagonal blocks (I + A_bb), column li per lane
@@ -994,7 +1021,32 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
       else
         v = c < 16 ? *reinterpret_cast<const f32x4*>(&sT[2][li][c])
                    : *reinterpret_cast<const f32x4*>(&sT[1][li][c - 16]);
-      *reinterpret_cast<f32x4*>(rec + R::kOffT + tid * 4) = v;
+      if constexpr (Heads)
+        put_planes(rec, HeadRecord::kT, 16 * w + li, c, v * *reinterpret_cast<const f32x4*>(&sBeta[c]));
+      else
+        *reinterpret_cast<f32x4*>(rec + R::kOffT + tid * 4) = v;
+    }
+    // P = P0 T, transposed (T^T P0^T), so that a lane's four results are four consecutive
+    // columns of row li of a tile: blocks (0, 0), (1, 0), (1, 1) by waves 0, 1, 2, and the zero
+    // block by wave 3; the summation index k = 4 lg + step as above
+    if constexpr (Heads) {
+      f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (wave < 3) {
+        const int mt = wave > 0 ? 1 : 0;
+        const int nt = wave > 1 ? 1 : 0;
+        const f32x4 p0 = *reinterpret_cast<const f32x4*>(&sP[member & 1][16 * mt + li][16 * nt + 4 * lg]);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) d = mfma(sT[nt][4 * lg + st][li], p0[st], d);
+        if (wave == 1) {   // + P0 (1, 1) T10
+          const f32x4 p1 = *reinterpret_cast<const f32x4*>(&sP[member & 1][16 + li][16 + 4 * lg]);
+#pragma unroll
+          for (int st = 0; st < 4; ++st) d = mfma(sT[2][4 * lg + st][li], p1[st], d);
+        }
+        d *= *reinterpret_cast<const f32x4*>(&sBeta[16 * nt + 4 * lg]);
+        put_planes(rec, HeadRecord::kP, 16 * mt + li, 16 * nt + 4 * lg, d);
+      } else {
+        put_planes(rec, HeadRecord::kP, li, 16 + 4 * lg, d);
+      }
     }
     // the next v-head writes -A after its first barrier (every read of -A and T above is
     // behind one of this v-head's) and its gates went to the other buffer
@@ -1016,51 +1068,6 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
 // all-fp32 products took 3,584.
 constexpr int kScanThreads = 512;
 
-// x = s1 + s2 + s3 exactly, in bf16 (each part the round-to-nearest-even of what the
-// earlier ones leave, and every remainder exact in fp32: 8 + 8 + 8 bits of x's 24), so a
-// product of an exact bf16 operand with x runs on the bf16 matrix cores as three products
-// with exact terms and fp32 sums.  p[i] holds part i + 1 of four values.
-struct Split4 {
-  uint2 p[3];
-};
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// two values to a packed bf16 pair (round to nearest even, one v_cvt_pk_bf16_f32)
-__device__ __forceinline__ uint32_t bf16_pair(f32x2 v) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-}
-
-// Each remainder r - s in one instruction: a dot product of the rounded pair with (-1, 0)
-// or (0, -1) added to r (v_dot2c_f32_bf16; exact products, and the sum is r - s, which
-// fp32 holds exactly).  (-1, 0) is set in an SGPR: as an operand the compiler encodes it
-// as the inline constant -1.0, which this instruction reads as the fp32 word 0xbf800000,
-// i.e. (0, -1).  Being an intrinsic, the first remainder also keeps a product passed as x
-// rounded to fp32 (x - s1 written out would be contracted into an fma of its factors).
-__device__ __forceinline__ Split4 split4(f32x4 x) {
-  Split4 sp;
-  uint32_t minus_lo_bits;
-  asm("s_mov_b32 %0, 0xbf80" : "=s"(minus_lo_bits));
-  const bf16x2 minus_lo = __builtin_bit_cast(bf16x2, minus_lo_bits);
-  const bf16x2 minus_hi = __builtin_bit_cast(bf16x2, 0xbf800000u);
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    f32x2 r = {x[2 * j], x[2 * j + 1]};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const uint32_t w = bf16_pair(r);
-      (j == 0 ? sp.p[i].x : sp.p[i].y) = w;
-      if (i < 2) {
-        const bf16x2 s = __builtin_bit_cast(bf16x2, w);
-        r = f32x2{__builtin_amdgcn_fdot2_f32_bf16(s, minus_lo, r.x, false),
-                  __builtin_amdgcn_fdot2_f32_bf16(s, minus_hi, r.y, false)};
-      }
-    }
-  }
-  return sp;
-}
-
 template <int RT>
 struct StateOperands {
   f32x4 w[8];      // W [16 w + li][32 lg + step]
@@ -1075,50 +1082,6 @@ struct OutputOperands {
   f32x4 sq;        // sq of tokens 16 w + 4 lg + r
   f32x4 p[4];      // P [16 w + li][16 lg + step]
 };
-
-// Buffer resource over one chunk record (raw, byte-addressed; word 3 = 0x00020000, the
-// gfx9 raw-buffer format) and a 16-byte load at lane offset + uniform offset: the address
-// stays a scalar resource plus one offset register, whatever the compiler's register
-// pressure.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t record_resource(const float* r, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(r), 0, bytes, 0x00020000);
-}
-
-// The state tile of (slot, head) as a buffer resource: over its 64 KiB when the sequence
-// starts from it, else over 0 bytes, whose loads return zeros without touching memory.  Its
-// loads then need no branch and go out together (a branch per load, as `from_slot ? load :
-// 0` compiles, waited for each load before the next was issued).  Callers pass the whole
-// offset per lane, so the range check sees all of it.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t state_resource(const DecodeParams& p, int slot,
-                                                                 int head, bool from_slot) {
-  // (uniform: readfirstlane keeps the resource in scalar registers, where a vector-held one
-  // would put each load in a loop over its distinct values)
-  return record_resource(
-      p.state + static_cast<int64_t>(slot) * p.state_slot + static_cast<int64_t>(head) * kDim * kDim,
-      __builtin_amdgcn_readfirstlane(from_slot ? kDim * kDim * 4 : 0));
-}
-
-// bf16 by the hardware's round-to-nearest-even conversion (v_cvt_pk_bf16_f32): the same
-// value as f32_to_bf16 for every finite input
-__device__ __forceinline__ uint16_t to_bf16(float f) {
-  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
-}
-
-__device__ __forceinline__ f32x4 load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t lane16,
-                                        int byte_offset) {
-  return __builtin_bit_cast(
-      f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(lane16), byte_offset, 0));
-}
-
-__device__ __forceinline__ u32x4 load16u(__amdgpu_buffer_rsrc_t rsrc, uint32_t lane16,
-                                         int byte_offset) {
-  return __builtin_bit_cast(
-      u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(lane16), byte_offset, 0));
-}
-
-__device__ __forceinline__ float load4(__amdgpu_buffer_rsrc_t rsrc, int byte_offset) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, 0, byte_offset, 0));
-}
 
 // The operand loads of one chunk come in pieces that the scan issues between its products,
 // a few at a time (issued in one burst at the top of a chunk, the CU's 116 loads would hold
@@ -1877,14 +1840,27 @@ int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
 // Workspace: the records, then chunk_start (num_sequences + 1 int32, rounded up to 256 B).
 // Sized for 64-token chunks, which covers 32-token ones: with S >= 1 sequences,
 // (T / 32 + S) R32 <= (2 (T / 64) + 1 + S) R32 <= (T / 64 + S) R64 as 2 R32 <= R64.
-static_assert(2 * Rec32::kSize <= kRecord, "32-token records fit the workspace");
+static_assert(2 * Rec32::kSize <= kRecord && HeadRecord::kBytes <= Rec32::kSize * 4,
+              "32-token records fit the workspace");
 int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
 }
 
+// Which scan the 32-token form runs: chunk_heads_kernel (a whole head per workgroup, norm
+// fused) or chunk_scan32_kernel (a head's rows over four workgroups).  A chunk takes a lone
+// workgroup of the first 3.5 us and of the second 2.3 us, so with few (sequence, head) pairs
+// the second's chain is the shorter; from two chunks per CU on the first's throughput decides,
+// and for prompts of one or two chunks the launch it saves (us, first / second, at 32 v-heads:
+// 1 x 64 27 / 28, 1 x 256 46 / 35, 4 x 256 50.9 / 49.8, 4 x 1024 144 / 137, 5 x 1024 150 / 181,
+// 8 x 128 41 / 50, 8 x 1024 179 / 258, 32 x 1024 625 / 985, 1024 x 32 1310 / 1710).
+bool whole_heads(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
+  return num_sequences * num_v_heads > 128 || num_tokens <= 64 * num_sequences;
+}
+
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
-                  float* ws, int32_t* chunk_start, hipStream_t stream) {
+                  bool w_bf16, float* ws, int32_t* chunk_start, hipStream_t stream,
+                  bool* normed) {
   constexpr int kCt = TT == 2 ? Rec32::kC : kC;
   const int64_t chunks = max_chunks<kCt>(num_tokens, num_sequences);
   if (chunks > 0x7fffffff || p.num_v_heads > 65535)
@@ -1895,32 +1871,42 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   const dim3 per_chunk(static_cast<uint32_t>(prep_groups));
   hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
                      num_sequences, chunk_start);
+  const bool heads = TT == 2 && whole_heads(num_tokens, num_sequences, p.num_v_heads);
+  *normed = heads;
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;
-#define LD_PREP_LAUNCH(K, D, W, N)                                                             \
-  hipLaunchKernelGGL((K<D, W>), per_chunk, dim3(N), 0, stream, p, num_sequences, ws,          \
+#define LD_PREP_LAUNCH(K, D, W, N, ...)                                                        \
+  hipLaunchKernelGGL((K<D, W __VA_OPT__(, ) __VA_ARGS__>), per_chunk, dim3(N), 0, stream, p, num_sequences, ws,          \
                      chunk_start, static_cast<int>(chunks))
-#define LD_PREP_LAUNCHES(K, N)                                                                 \
+#define LD_PREP_LAUNCHES(K, N, ...)                                                            \
   if (dt_bf16) {                                                                               \
     if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, true, true, N);                                                        \
+      LD_PREP_LAUNCH(K, true, true, N, __VA_ARGS__);                                                        \
     else                                                                                       \
-      LD_PREP_LAUNCH(K, true, false, N);                                                       \
+      LD_PREP_LAUNCH(K, true, false, N, __VA_ARGS__);                                                       \
   } else {                                                                                     \
     if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, false, true, N);                                                       \
+      LD_PREP_LAUNCH(K, false, true, N, __VA_ARGS__);                                                       \
     else                                                                                       \
-      LD_PREP_LAUNCH(K, false, false, N);                                                      \
+      LD_PREP_LAUNCH(K, false, false, N, __VA_ARGS__);                                                      \
   }
   if constexpr (TT == 2) {
-    LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads)
+    if (heads) {
+      LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads, true)
+    } else {
+      LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads, false)
+    }
   } else {
     LD_PREP_LAUNCHES(chunk_prep_kernel, kPrepThreads)
   }
 #undef LD_PREP_LAUNCHES
 #undef LD_PREP_LAUNCH
   const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
-  if constexpr (TT == 2) {
+  if (heads) {
+    const int rc = launch_chunk_heads(p, num_sequences, ws, chunk_start, static_cast<int>(chunks),
+                                      w_bf16, stream);
+    if (rc != LD_OK) return rc;
+  } else if constexpr (TT == 2) {
     const int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
     if (scan_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
     hipLaunchKernelGGL(chunk_scan32_kernel, dim3(static_cast<uint32_t>(scan_groups)),
@@ -1952,13 +1938,16 @@ int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequence
 }
 
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
-                           bool dt_bf16, int chunk_tokens, void* workspace, hipStream_t stream) {
+                           bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
+                           hipStream_t stream, bool* normed) {
   float* ws = static_cast<float*>(workspace);
   int32_t* chunk_start = reinterpret_cast<int32_t*>(
       static_cast<char*>(workspace) + records_bytes(num_tokens, num_sequences, p.num_v_heads));
   if (chunk_tokens == 32)
-    return launch_chunks<2>(p, num_sequences, num_tokens, dt_bf16, ws, chunk_start, stream);
-  return launch_chunks<4>(p, num_sequences, num_tokens, dt_bf16, ws, chunk_start, stream);
+    return launch_chunks<2>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start,
+                            stream, normed);
+  return launch_chunks<4>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start, stream,
+                          normed);
 }
 
 }  // namespace ld

@@ -1,0 +1,657 @@
+// Chunked prefill for gfx950, 32-token chunks, one workgroup per (sequence, v-head): the scan
+// of prefill_chunked.hip's 32-token form with the whole head's state in registers and the
+// gated RMSNorm fused in.
+//
+// Four waves; wave w owns state rows v = 32 w .. 32 w + 31 as S^T in the accumulator layout of
+// v_mfma_f32_32x32x16_bf16 (fp32, 64 registers).  For lane l, lj = l % 32 and hi = l / 32; a
+// 32 x 32 accumulator holds rows i(r) = 8 (r / 4) + 4 hi + r % 4, r < 16, of column lj, and an
+// operand A[i = lj][k = 8 hi + e] or B[k = 8 hi + e][j = lj], e < 8.  The summation index may
+// be assigned to (step, hi, e) freely as long as both operands agree, so an accumulator's
+// registers 8 u .. 8 u + 7 are directly the B operand of step u once split into bf16 planes:
+// nothing of the chain S -> Y -> X -> V_new -> S' moves between lanes or waves.
+//   state tile T < 4:  row i of the accumulator is k = 32 T + key_of(i), chosen so that step u
+//                      takes k = 32 T + 16 u + 8 hi + e: 16 consecutive bytes of a q or k row
+//   tokens:            row i of an accumulator over the chunk is token i, so step u of a
+//                      product over tokens takes token 16 u + 8 (e / 4) + 4 hi + e % 4
+// Per chunk and wave (rows past the sequence's end are zeros):
+//   Y = K S^T, O = Q S^T    (q, k as stored against S's exact three-way split: 24 products each)
+//   X = V - diag(ws) Y
+//   V_new = T X             (T = (I + A)^-1 diag(beta); six products of planes: all but those
+//                           below 2^-26 of |T| |X|)
+//   O = diag(sq) O + P X    (P = P0 T: P0 V_new without waiting for V_new; the same)
+//   S' = exp(G_n-1) S + K^T (ck V_new)   (24 products)
+// and the chunk's raw outputs go through LDS (bf16, the reference's rounding point) to the
+// gated RMSNorm of whole rows.  q, k and v come from qkv through LDS, the transposed operands
+// by ds_read_b64_tr_b16; T, P (as planes) and the per-token scales from the prep's records.
+//
+// What bounds it: the matrix pipe and the vector work of the splits.  A wave's chunk is 96
+// matrix instructions (3,072 cycles) and, with the norm, 690 vector ones, of which the 192
+// v_dot2 run alone (8 of them behind a matrix instruction took 78 cycles, 8 multiply-adds 43,
+// 6 of those 34), so about 4,200 cycles; two workgroups a CU take 4,800 per head and chunk.  At
+// 32 x 1024 tokens and 32 v-heads that is 0.94 PFLOP/s of bf16 products at a clock that the
+// card's power limit holds at 1.6 GHz (a large bf16 GEMM reaches 1.17), 438 us, where
+// chunk_scan32_kernel and the norm pass took 820 us: with a head's rows over four workgroups
+// every wave re-read S's planes from LDS and the raw outputs crossed HBM twice more.  The whole
+// prefill went from 985 to 625 us there, 257 to 179 us at 8 x 1024, 1,710 to 1,310 us at
+// 1024 x 32.  Products and vector work are laid out by hand, slot by slot: as the compiler
+// scheduled the same code, 32 x 1024 took 685 us.
+#include "chunk_common.h"
+
+namespace ld {
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTok = HeadRecord::kTokens;
+constexpr int kTileRow = kDim * 2;             // bytes of a q, k, v or raw-output row in LDS
+constexpr int kTileSize = kTok * kTileRow;
+
+// 16-byte pieces of row r are stored at piece ^ swizzle(r): a column of pieces over 16 rows
+// (operand A of the products with S) and 4 x 4 element blocks of 4 rows (transposed reads)
+// each cover every bank once.
+__device__ __forceinline__ constexpr int swizzle(int row) {
+  return ((row & 3) << 2) | ((row >> 2) & 3);
+}
+
+__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Fixes the order of pure operations: a value is defined ahead of this point and not used
+// before it, and the points keep their order in the program.  (Left to itself the compiler
+// lines the splits up ahead of the matrix instructions that should run beside them; it
+// emits nothing for a pin.)
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+// r - s for a pair of values and its rounded bf16 pair, both for four pairs: each value plus
+// the dot product of the pair with (-1, 0) or (0, -1), exact as in split4, but with the
+// three-operand form, which leaves r in place (the builtin's two-operand form costs a move per
+// value that lives on, as the state does).  The dots' results are ready for any instruction
+// three issue slots later: the block ends with the wait.
+__device__ __forceinline__ void remainders(const float (&r)[8], u32x4 w, float (&out)[8]) {
+  const uint32_t w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+  asm volatile(
+      "v_dot2_f32_bf16 %0, %16, %20, %8\n\t"
+      "v_dot2_f32_bf16 %1, %16, %21, %9\n\t"
+      "v_dot2_f32_bf16 %2, %17, %20, %10\n\t"
+      "v_dot2_f32_bf16 %3, %17, %21, %11\n\t"
+      "v_dot2_f32_bf16 %4, %18, %20, %12\n\t"
+      "v_dot2_f32_bf16 %5, %18, %21, %13\n\t"
+      "v_dot2_f32_bf16 %6, %19, %20, %14\n\t"
+      "v_dot2_f32_bf16 %7, %19, %21, %15\n\t"
+      "s_nop 2"
+      : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3]), "=&v"(out[4]), "=&v"(out[5]),
+        "=&v"(out[6]), "=&v"(out[7])
+      : "v"(r[0]), "v"(r[1]), "v"(r[2]), "v"(r[3]), "v"(r[4]), "v"(r[5]), "v"(r[6]), "v"(r[7]),
+        "v"(w0), "v"(w1), "v"(w2), "v"(w3), "s"(0x0000bf80u), "s"(0xbf800000u));
+}
+
+// The exact split of eight values (a lane's registers 8 u .. 8 u + 7 of an accumulator) into
+// planes that are B operands, in five stages of 4 or 8 instructions: a stage fits beside one
+// matrix instruction.
+struct Split8 {
+  float r[8];
+  u32x4 w[3];
+  __device__ __forceinline__ void set(f32x4 lo, f32x4 hi) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[e] = lo[e];
+      r[4 + e] = hi[e];
+    }
+  }
+  __device__ __forceinline__ void stage(int i) {  // 0 .. 4
+    if (i & 1) {
+      float rest[8];
+      remainders(r, w[i >> 1], rest);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = rest[e];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[i >> 1][j] = bf16_pair(f32x2{r[2 * j], r[2 * j + 1]});
+      pin(w[i >> 1]);
+    }
+  }
+  __device__ __forceinline__ void all() {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) stage(i);
+  }
+  __device__ __forceinline__ bf16x8 plane(int i) const {
+    return __builtin_bit_cast(bf16x8, w[i]);
+  }
+};
+__device__ __forceinline__ f32x4 quad(const f32x16& x, int q) {
+  return f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+}
+
+// A matrix instruction in its place of the schedule (First: of a sum that starts at zero).
+template <bool First = false>
+__device__ __forceinline__ void product(bf16x8 a, bf16x8 b, f32x16& c) {
+  if constexpr (First) {
+    pin(a);
+    c = mfma32(a, b, f32x16{});
+  } else {
+    pin(c);
+    c = mfma32(a, b, c);
+  }
+  pin(c);
+}
+
+// 4 x 16 block of bf16 transposed on the way from LDS: within 16 lanes, lane m gives the
+// address of row m / 4, elements 4 (m % 4) .. + 3, and receives rows 0 .. 3 of column m.
+__device__ __forceinline__ bf16x4 read_tr(const uint8_t* at) {
+  const auto p = (__attribute__((address_space(3))) s16x4*)(at);
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p));
+}
+
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Sixteen bytes of a row at a lane's byte offset + a uniform one: one load, or (rows not at
+// 16-byte boundaries) eight of one element.
+template <bool Wide>
+__device__ __forceinline__ u32x4 load_piece(__amdgpu_buffer_rsrc_t rs, uint32_t offset,
+                                            int uniform) {
+  if constexpr (Wide) return load16u(rs, offset, uniform);
+  u32x4 out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b16(rs, static_cast<int>(offset + 4 * i), uniform, 0);
+    const uint32_t hi = __builtin_amdgcn_raw_buffer_load_b16(rs, static_cast<int>(offset + 4 * i + 2), uniform, 0);
+    out[i] = (lo & 0xffffu) | (hi << 16);
+  }
+  return out;
+}
+
+// The gated RMSNorm of a chunk's rows, a thread's 16 columns of one token, in slices that fit
+// beside matrix instructions: 0: the raw outputs' reads, 1-4: squares, 5: the row's sum over its
+// 8 threads, 6: rstd, 7-22: two per pair of columns.  Arithmetic as prefill_norm_kernel's.
+struct Norm {
+  u32x4 raw[2], gate[2], y[2];
+  float ss, rstd, sig0, sig1;
+  f32x2 w;
+  __device__ __forceinline__ void slice(int i, const uint8_t* raw0, const uint8_t* raw1,
+                                        const float* weight, float eps) {
+    if (i == 0) {
+      raw[0] = *reinterpret_cast<const u32x4*>(raw0);
+      raw[1] = *reinterpret_cast<const u32x4*>(raw1);
+      ss = 0.0f;
+    } else if (i < 5) {
+#pragma unroll
+      for (int d = 2 * ((i - 1) & 1); d < 2 * ((i - 1) & 1) + 2; ++d) {
+        const uint32_t bits = raw[(i - 1) >> 1][d];
+        const float lo = __builtin_bit_cast(float, bits << 16);
+        const float hi = __builtin_bit_cast(float, bits & 0xffff0000u);
+        ss = fmaf(lo, lo, ss);
+        ss = fmaf(hi, hi, ss);
+      }
+      pin(ss);
+    } else if (i == 5) {
+      ss += dpp<kDppQuadXor1>(ss);
+      ss += dpp<kDppQuadXor2>(ss);
+      ss += dpp<kDppRowHalfMirror>(ss);
+      pin(ss);
+    } else if (i == 6) {
+      rstd = fast_rsqrt(ss / static_cast<float>(kDim) + eps);
+      pin(rstd);
+    } else {
+      const int j = (i - 7) >> 1;   // pair of columns
+      const uint32_t gb = gate[j >> 2][j & 3];
+      const float g0 = __builtin_bit_cast(float, gb << 16);
+      const float g1 = __builtin_bit_cast(float, gb & 0xffff0000u);
+      if ((i - 7) % 2 == 0) {
+        w = *reinterpret_cast<const f32x2*>(weight + 2 * j);
+        sig0 = sigmoid(g0);
+        sig1 = sigmoid(g1);
+        pin(sig0);
+        pin(sig1);
+      } else {
+        const uint32_t rb = raw[j >> 2][j & 3];
+        const float y0 =
+            ((__builtin_bit_cast(float, rb << 16) * rstd) * w.x) * (g0 * sig0);
+        const float y1 =
+            ((__builtin_bit_cast(float, rb & 0xffff0000u) * rstd) * w.y) * (g1 * sig1);
+        y[j >> 2][j & 3] = bf16_pair(f32x2{y0, y1});
+        pin(y[j >> 2]);
+      }
+    }
+  }
+};
+
+// Wide: the rows of qkv, gate and out start at 16-byte boundaries.
+template <bool WBf16, bool Wide>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws,
+                        const int32_t* chunk_start, int records) {
+  using R = HeadRecord;
+  // Workgroups go to the 8 XCDs round-robin by id; the v-heads of one (sequence, k-head) read
+  // the same q and k, so they are given ids on one XCD.
+  const int xcd = blockIdx.x & 7;
+  const int rank = blockIdx.x >> 3;
+  const int unit = (rank / p.group) * 8 + xcd;
+  if (unit >= num_sequences * p.num_k_heads) return;
+  const int seq = unit / p.num_k_heads;
+  const int key_head = unit - seq * p.num_k_heads;
+  const int head = key_head * p.group + rank % p.group;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lj = lane & 31;
+  const int hi = lane >> 5;
+  const int bos = p.cu[seq];
+  const int eos = p.cu[seq + 1];
+  const int slot = p.indices[seq];
+  const bool from_slot = slot > 0 && p.has_initial[seq] != 0;
+  const int gbase = chunk_start[seq];
+  // (bounded by the records the workspace holds, whatever cu_seqlens says)
+  const int chunks = min((eos - bos + kTok - 1) / kTok, max(records - gbase, 0));
+
+  __shared__ __attribute__((aligned(16))) uint8_t sK[kTileSize];
+  __shared__ __attribute__((aligned(16))) uint8_t sQ[kTileSize];
+  // v of the chunk, then in its place the raw outputs (a wave reads and writes its own 32
+  // columns of both); two, as the norm reads one while the next chunk's v arrives
+  __shared__ __attribute__((aligned(16))) uint8_t sV[2][kTileSize];
+  __shared__ __attribute__((aligned(16))) uint8_t sRec[R::kBytes];
+  __shared__ float sW[kDim];
+
+  if (tid < kDim) sW[tid] = load_param(p.norm_weight, tid, WBf16);
+
+  // ---- operands of one chunk, in registers on their way to LDS ----
+  const uint32_t row_bytes = static_cast<uint32_t>(p.qkv_row) * 2;
+  const int srow = tid >> 4;         // row (+ 16 for the second piece) and piece of this thread
+  const int spiece = tid & 15;
+  const uint32_t src = srow * row_bytes + spiece * 16;
+  const int q_col = key_head * kTileRow;
+  const int k_col = (p.num_k_heads + key_head) * kTileRow;
+  const int v_col = (2 * p.num_k_heads + head) * kTileRow;
+  const int qkv_bytes = (2 * p.num_k_heads + p.num_v_heads) * kTileRow;
+  const uint32_t dst = srow * kTileRow + ((spiece ^ swizzle(srow)) << 4);
+  struct Staged {
+    u32x4 q[2], k[2], v[2], rec[3];
+    uint32_t scales;
+  };
+  // Where chunk c's operands are (past the last chunk: resources over 0 bytes, whose loads
+  // return zeros), and its load i of 10.
+  struct Source {
+    __amdgpu_buffer_rsrc_t rows, rec;
+    uint32_t at[2];
+  };
+  auto source = [&](int c) __attribute__((always_inline)) {
+    Source x;
+    const int t0 = bos + min(c, max(chunks - 1, 0)) * kTok;
+    const int live = c < chunks ? min(kTok, eos - t0) : 0;   // rows of the chunk
+    x.rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.qkv + static_cast<int64_t>(t0) * p.qkv_row), 0,
+        live > 0 ? (live - 1) * static_cast<int>(row_bytes) + qkv_bytes : 0, 0x00020000);
+    x.rec = record_resource(
+        ws + (static_cast<int64_t>(gbase + min(c, max(chunks - 1, 0))) * p.num_v_heads + head) *
+                 (R::kBytes / 4),
+        c < chunks ? R::kBytes : 0);
+    // rows past the chunk's end: an offset past the resource, so zeros
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x.at[i] = srow + 16 * i < live ? src + i * 16 * row_bytes : 0xfffff000u;
+    return x;
+  };
+  auto fetch = [&](Staged& x, const Source& from, int i) __attribute__((always_inline)) {
+    if (i < 2)
+      x.k[i] = load_piece<Wide>(from.rows, from.at[i], k_col);
+    else if (i < 4)
+      x.q[i - 2] = load_piece<Wide>(from.rows, from.at[i - 2], q_col);
+    else if (i < 6)
+      x.v[i - 4] = load_piece<Wide>(from.rows, from.at[i - 4], v_col);
+    else if (i < 9)
+      x.rec[i - 6] = load16u(from.rec, tid * 16 + (i - 6) * 4096, 0);
+    else
+      x.scales = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + R::kScales, 0, 0);
+  };
+  auto put = [&](const Staged& x, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      *reinterpret_cast<u32x4*>(sK + dst + i * 16 * kTileRow) = x.k[i];
+      *reinterpret_cast<u32x4*>(sQ + dst + i * 16 * kTileRow) = x.q[i];
+      *reinterpret_cast<u32x4*>(sV[buf] + dst + i * 16 * kTileRow) = x.v[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(sRec + tid * 16 + i * 4096) = x.rec[i];
+    if (tid < (R::kBytes - R::kScales) / 4)
+      *reinterpret_cast<uint32_t*>(sRec + tid * 4 + R::kScales) = x.scales;
+  };
+  static_assert(R::kScales == 3 * 4096 && R::kBytes - R::kScales <= kThreads * 4,
+                "three pieces and a scale per thread");
+
+  Staged staged;
+  if (chunks > 0) {
+    const Source from = source(0);
+#pragma unroll
+    for (int i = 0; i < 10; ++i) fetch(staged, from, i);
+  }
+
+  // st[T][8 u + 4 h + r] = S[32 w + lj][32 T + 16 u + 8 hi + 4 h + r]
+  f32x16 st[4];
+  {
+    const __amdgpu_buffer_rsrc_t srs = state_resource(p, slot, head, from_slot);
+    const uint32_t at = static_cast<uint32_t>(((32 * w + lj) * kDim + 8 * hi) * 4);
+#pragma unroll
+    for (int T = 0; T < 4; ++T)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 x = load16(srs, at + (32 * T + 16 * (q >> 1) + 4 * (q & 1)) * 4, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) st[T][4 * q + r] = x[r];
+      }
+  }
+
+  // lane addresses of the operands (the swizzle's parts that depend on the step are XORed in)
+  const uint32_t a_at = lj * kTileRow + ((hi ^ swizzle(lj)) << 4);       // ^ ((4 T + 2 u) << 4)
+  const int m = lane & 15;
+  const int c16 = (lane >> 4) & 1;
+  const uint32_t tr_row = (4 * hi + (m >> 2)) * kTileRow;
+  // transposed k: rows 16 u + 8 h + .., columns key_of(16 c16 + ..)   ^ (T << 6) ^ (h << 5)
+  const uint32_t kt_at =
+      tr_row + (((2 * c16 + (m & 1)) ^ ((m >> 2) << 2) ^ hi) << 4) + ((m >> 1) & 1) * 8;
+  // transposed v: rows 8 q + .., the wave's columns   ^ ((q & 1) << 5)
+  const uint32_t vt_at =
+      tr_row + (((4 * w + 2 * c16 + ((m & 3) >> 1)) ^ ((m >> 2) << 2) ^ hi) << 4) + (m & 1) * 8;
+  // raw outputs: row 8 q + 4 hi + e, column 32 w + lj   ^ (e << 6) ^ ((q & 1) << 5)
+  const uint32_t raw_at =
+      4 * hi * kTileRow + (((4 * w + (lj >> 3)) ^ hi) << 4) + (lj & 7) * 2;
+  const uint8_t* const planes = sRec + lane * 16;
+  const f32x4* const scales = reinterpret_cast<const f32x4*>(sRec + R::kScales) + hi;
+
+  // The norm of chunk c - 1 runs beside chunk c's products; thread = (token, 16 columns).
+  // Resources over the chunk's rows of gate and out (before the first chunk: over 0 bytes,
+  // whose loads return zeros and whose stores are dropped).
+  const int ntok = tid >> 3;
+  const int ncol = (tid & 7) * 16;
+  const uint32_t gate_bytes = static_cast<uint32_t>(p.gate_row) * 2;
+  const uint32_t out_bytes = static_cast<uint32_t>(p.num_v_heads) * kTileRow;
+  const uint32_t raw0_at = ntok * kTileRow + (((ncol >> 3) ^ swizzle(ntok)) << 4);
+  const uint32_t raw1_at = ntok * kTileRow + ((((ncol >> 3) + 1) ^ swizzle(ntok)) << 4);
+  auto chunk_rows = [&](const uint16_t* base, int64_t row, int c) __attribute__((always_inline)) {
+    const int t0 = bos + max(c, 0) * kTok;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(base + static_cast<int64_t>(t0) * row + static_cast<int64_t>(head) * kDim),
+        0, c >= 0 ? (min(kTok, eos - t0) - 1) * static_cast<int>(row * 2) + kTileRow : 0, 0x00020000);
+  };
+  auto load_gate = [&](Norm& norm, int c) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rows = chunk_rows(p.gate, p.gate_row, c);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      norm.gate[i] = load_piece<Wide>(rows, ntok * gate_bytes + ncol * 2 + 16 * i, 0);
+  };
+  auto store_norm = [&](const Norm& norm, int c) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rows = chunk_rows(p.out, static_cast<int64_t>(p.num_v_heads) * kDim, c);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int at = static_cast<int>(ntok * out_bytes) + ncol * 2 + 16 * i;
+      if constexpr (Wide) {
+        __builtin_amdgcn_raw_buffer_store_b128(norm.y[i], rows, at, 0, 0);
+      } else {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(norm.y[i][d]), rows, at + 4 * d, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(norm.y[i][d] >> 16), rows, at + 4 * d + 2, 0, 0);
+        }
+      }
+    }
+  };
+
+  // (the state's loads are waited for here: inside the loop the waits would be counted
+  // against later chunks' loads)
+#pragma unroll
+  for (int T = 0; T < 4; ++T) pin(st[T]);
+  for (int c = 0; c < chunks; ++c) {
+    const int buf = c & 1;
+    put(staged, buf);
+    lds_barrier();   // the chunk's operands and the previous chunk's raw outputs are in LDS
+
+    // The next chunk's loads go out between the products below (a burst of them holds the wave
+    // until the last is accepted, and in registers before they are due).
+    const Source from = source(c + 1);
+    auto prefetch = [&](int i) __attribute__((always_inline)) {
+      asm volatile("" ::: "memory");
+      fetch(staged, from, i);
+      asm volatile("" ::: "memory");
+    };
+    Norm norm;
+    load_gate(norm, c - 1);
+    const uint8_t* const last_raw = sV[buf ^ 1];
+    auto normalise = [&](int i) __attribute__((always_inline)) {
+      norm.slice(i, last_raw + raw0_at, last_raw + raw1_at, sW + ncol, p.eps);
+    };
+
+    // Y = K S^T and O = Q S^T: step n = 2 T + u takes k = 32 T + 16 u + ..; beside its products
+    // the next step's operands are read and its S split, and S is scaled once split.  The last
+    // two steps' O products come after Y's, beside X = V - diag(ws) Y (ws and v are zero past
+    // the sequence's end) and its split.
+    f32x16 y, o;
+    auto operand = [&](const uint8_t* tile, int n) __attribute__((always_inline)) {
+      return *reinterpret_cast<const bf16x8*>(tile + (a_at ^ (n << 5)));
+    };
+    const float gamma = *reinterpret_cast<const float*>(sRec + R::kGamma);
+    Split8 now, next, held;
+    bf16x8 ka = operand(sK, 0), qa = operand(sQ, 0), q6;
+    now.set(quad(st[0], 0), quad(st[0], 1));
+    now.all();
+    bf16x4 vt[4];
+    f32x4 wsc[4], xs[4];
+    auto scale_state = [&](int T, int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 8 * u; e < 8 * u + 8; ++e) st[T][e] *= gamma;
+      pin(st[T]);
+    };
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const bf16x8 kc = ka, qc = qa;
+      if (n == 1 || n == 3 || n == 5) prefetch(n >> 1);
+      if (n < 7) {
+        ka = operand(sK, n + 1);
+        qa = operand(sQ, n + 1);
+        next.set(quad(st[(n + 1) >> 1], 2 * ((n + 1) & 1)), quad(st[(n + 1) >> 1], 2 * ((n + 1) & 1) + 1));
+      }
+      if (n < 6) {
+        if (n == 0) product<true>(kc, now.plane(2), y); else product(kc, now.plane(2), y);
+        next.stage(0);
+        if (n == 0) product<true>(qc, now.plane(2), o); else product(qc, now.plane(2), o);
+        next.stage(1);
+        product(kc, now.plane(1), y);
+        next.stage(2);
+        product(qc, now.plane(1), o);
+        next.stage(3);
+        product(kc, now.plane(0), y);
+        next.stage(4);
+        product(qc, now.plane(0), o);
+        if (n > 0) scale_state((n - 1) >> 1, (n - 1) & 1);
+        now = next;
+      } else if (n == 6) {
+        product(kc, now.plane(2), y);
+        next.stage(0);
+        next.stage(1);
+        product(kc, now.plane(1), y);
+        next.stage(2);
+        next.stage(3);
+        product(kc, now.plane(0), y);
+        next.stage(4);
+        held = now;
+        q6 = qc;
+        now = next;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          vt[q] = read_tr(sV[buf] + (vt_at ^ ((q & 1) << 5)) + 8 * q * kTileRow);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) wsc[q] = scales[R::kWs + 2 * q];
+        product(kc, now.plane(2), y);
+        scale_state(2, 1);
+        product(kc, now.plane(1), y);
+        scale_state(3, 0);
+        product(kc, now.plane(0), y);
+        scale_state(3, 1);
+        product(q6, held.plane(2), o);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) xs[q][r] = static_cast<float>(vt[q][r]);
+          pin(xs[q]);
+        }
+        product(q6, held.plane(1), o);
+        product(q6, held.plane(0), o);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) xs[q][r] = fmaf(-wsc[q][r], y[4 * q + r], xs[q][r]);
+          pin(xs[q]);
+        }
+        held.set(xs[0], xs[1]);
+        next.set(xs[2], xs[3]);
+        held.stage(0);
+        held.stage(1);
+        product(qc, now.plane(2), o);
+        held.stage(2);
+        product(qc, now.plane(1), o);
+        held.stage(3);
+        product(qc, now.plane(0), o);
+        held.stage(4);
+      }
+    }
+    // V_new = T X and O = diag(sq) O + P X, T and P as planes (held, next: X's), the smallest
+    // products of a step first
+    auto weight = [&](int base, int u, int i) __attribute__((always_inline)) {
+      return *reinterpret_cast<const bf16x8*>(planes + base + (3 * u + i) * 1024);
+    };
+    // the six products of a step; NEXT, UN: the matrix and step whose planes replace the
+    // current ones as they fall free
+#define LD_PRODUCTS(FIRST, ACC, X, SLOT, NEXT, UN)                                            \
+  product<FIRST>(wt[2], X.plane(0), ACC); wt[2] = weight(NEXT, UN, 2); SLOT(0);               \
+  product(wt[1], X.plane(1), ACC); SLOT(1);                                                   \
+  product(wt[0], X.plane(2), ACC); SLOT(2);                                                   \
+  product(wt[1], X.plane(0), ACC); wt[1] = weight(NEXT, UN, 1); SLOT(3);                      \
+  product(wt[0], X.plane(1), ACC); SLOT(4);                                                   \
+  product(wt[0], X.plane(0), ACC); wt[0] = weight(NEXT, UN, 0); SLOT(5);
+    f32x16 vn;
+    bf16x8 wt[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) wt[i] = weight(R::kT, 0, i);
+    f32x4 sq[4], ck[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sq[q] = scales[R::kSq + 2 * q];
+    auto slot_t0 = [&](int i) __attribute__((always_inline)) {
+      if (i < 5) next.stage(i);
+      if (i % 2 == 0) prefetch(3 + i / 2);
+    };
+    LD_PRODUCTS(true, vn, held, slot_t0, R::kT, 1)
+    auto slot_t1 = [&](int i) __attribute__((always_inline)) {
+      if (i < 2) {
+#pragma unroll
+        for (int q = 2 * i; q < 2 * i + 2; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[4 * q + r] *= sq[q][r];
+        pin(o);
+      } else {
+        normalise(i - 2);
+      }
+    };
+    LD_PRODUCTS(false, vn, next, slot_t1, R::kP, 0)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) ck[q] = scales[R::kCk + 2 * q];
+    // beside P X: the split of ck V_new (now: step 0, last: step 1)
+    Split8 last;
+    auto slot_p0 = [&](int i) __attribute__((always_inline)) {
+      if (i % 3 == 0) prefetch(6 + i / 3);
+      if (i == 0) {
+        normalise(4);
+      } else if (i == 1) {
+        now.set(quad(vn, 0) * ck[0], quad(vn, 1) * ck[1]);
+        now.stage(0);
+      } else {
+        now.stage(i - 1);
+      }
+      if (i >= 4) ck[i - 2] = scales[R::kCk + 2 * (i - 2)];
+    };
+    LD_PRODUCTS(false, o, held, slot_p0, R::kP, 1)
+    auto slot_p1 = [&](int i) __attribute__((always_inline)) {
+      if (i % 3 == 0) prefetch(8 + i / 3);
+      if (i == 0)
+        last.set(quad(vn, 2) * ck[2], quad(vn, 3) * ck[3]);
+      else
+        last.stage(i - 1);
+    };
+    LD_PRODUCTS(false, o, next, slot_p1, R::kP, 1)
+#undef LD_PRODUCTS
+    // S' = exp(G_n-1) S + K^T (ck V_new); beside it the raw outputs to LDS, rounded to bf16, and
+    // the previous chunk's norm
+    auto key_t = [&](int i) __attribute__((always_inline)) {   // tile i % 4, step i / 4
+      const int T = i & 3, u = i >> 2;
+      const bf16x4 k0 = read_tr(sK + (kt_at ^ (T << 6)) + 16 * u * kTileRow);
+      const bf16x4 k1 = read_tr(sK + (kt_at ^ (T << 6) ^ (1 << 5)) + (16 * u + 8) * kTileRow);
+      return __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    bf16x8 kt = key_t(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bf16x8 kc = kt;
+      if (i < 7) kt = key_t(i + 1);
+#pragma unroll
+      for (int pl = 2; pl >= 0; --pl) {
+        product(kc, i < 4 ? now.plane(pl) : last.plane(pl), st[i & 3]);
+        const int n = 3 * i + 2 - pl;   // 0 .. 23
+        if (n < 2) normalise(5 + n);
+        else if (n >= 4 && n < 20) normalise(n + 3);
+        if (n >= 2 && n % 3 == 2) {   // two tokens in each of eight slots
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int tok = 2 * ((n - 2) / 3) + e, q = tok >> 2;
+            *reinterpret_cast<uint16_t*>(sV[buf] + (raw_at ^ ((tok & 3) << 6) ^ ((q & 1) << 5)) +
+                                         (8 * q + (tok & 3)) * kTileRow) = to_bf16(o[tok]);
+          }
+        }
+      }
+    }
+    store_norm(norm, c - 1);
+    lds_barrier();   // every read of the operands is done
+  }
+  if (chunks > 0) {   // the last chunk's norm (its raw outputs are complete past the barrier)
+    Norm norm;
+    load_gate(norm, chunks - 1);
+    const uint8_t* const last_raw = sV[(chunks - 1) & 1];
+#pragma unroll
+    for (int i = 0; i < 23; ++i)
+      norm.slice(i, last_raw + raw0_at, last_raw + raw1_at, sW + ncol, p.eps);
+    store_norm(norm, chunks - 1);
+  }
+
+  if (slot > 0) {
+    float* tile = p.state + static_cast<int64_t>(slot) * p.state_slot +
+                  static_cast<int64_t>(head) * kDim * kDim + (32 * w + lj) * kDim + 8 * hi;
+#pragma unroll
+    for (int T = 0; T < 4; ++T)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(tile + 32 * T + 16 * (q >> 1) + 4 * (q & 1)) = quad(st[T], q);
+  }
+}
+
+}  // namespace
+
+int launch_chunk_heads(const DecodeParams& p, int num_sequences, const float* ws,
+                       const int32_t* chunk_start, int records, bool w_bf16, hipStream_t stream) {
+  const int64_t units = static_cast<int64_t>(num_sequences) * p.num_k_heads;
+  const int64_t groups = (units + 7) / 8 * 8 * p.group;
+  if (groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
+  const auto at16 = [](const void* base, int64_t row) {
+    return (reinterpret_cast<uintptr_t>(base) & 15) == 0 && (row & 7) == 0;
+  };
+  const bool wide = at16(p.qkv, p.qkv_row) && at16(p.gate, p.gate_row) && at16(p.out, 0);
+  const auto kernel = w_bf16 ? (wide ? chunk_heads_kernel<true, true> : chunk_heads_kernel<true, false>)
+                             : (wide ? chunk_heads_kernel<false, true> : chunk_heads_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(kThreads), 0, stream, p,
+                     num_sequences, ws, chunk_start, records);
+  return LD_OK;
+}
+
+}  // namespace ld

@@ -534,9 +534,10 @@ int prefill(const ld_gdn_prefill_args& a, void* workspace, int64_t workspace_byt
           : 0;
   const bool chunked = chunk_tokens != 0;
   if (chunked) {
-    const int rc = launch_prefill_chunked(p, a.num_sequences, a.num_tokens, dt_bf16,
-                                          chunk_tokens, workspace, s);
-    if (rc != LD_OK) return rc;
+    bool normed = false;
+    const int rc = launch_prefill_chunked(p, a.num_sequences, a.num_tokens, dt_bf16, w_bf16,
+                                          chunk_tokens, workspace, s, &normed);
+    if (rc != LD_OK || normed) return rc;
   }
   // Token-serial: split a head's rows over more workgroups when (sequence, head) tiles alone
   // would leave the GPU short of work (1024 tiles fill 256 CUs at 4 per CU).

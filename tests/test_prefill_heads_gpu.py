@@ -1,0 +1,90 @@
+"""The 32-token chunked prefill with a whole head per workgroup (csrc/prefill_heads.hip): prompt
+lengths at the edges of its chunks, every head grouping, both sides of the rule that picks it,
+and rows of gate and qkv that start at no 16-byte boundary, against the oracle (the parity
+helpers' tolerances)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from lightdelta_amd import ops
+from oracle.decode import expected_prefill
+from tests.parity import assert_bf16_outputs, assert_states
+from tests.test_prefill_gpu import PREFILL, announce, prefill_case, run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def chunked_32():
+    saved = ops.prefill_algorithm()
+    ops.set_prefill_algorithm("chunked_32")
+    yield
+    ops.set_prefill_algorithm(saved)
+
+
+def check(case):
+    exp_out, exp_pool, pre = expected_prefill(*[case[k] for k in PREFILL], 1e-6, return_pre=True)
+    before = case["pool"].clone()
+    run(case)
+    torch.cuda.synchronize()
+    assert_bf16_outputs(case["out"], exp_out, pre)
+    assert_states(case["pool"], exp_pool)
+    assert torch.equal(case["pool"][0], before[0])
+
+
+@pytest.mark.parametrize("heads", [(1, 1), (2, 6), (16, 16), (4, 32), (16, 48)])
+def test_chunk_edges(gpu, heads):
+    """Lengths one below, at and above one, two and three chunks, one token, none; zero and
+    given initial states; a padding slot."""
+    lengths = [1, 31, 32, 33, 0, 63, 64, 65, 96, 97, 2]
+    announce(test="heads_chunk_edges", heads=heads, lengths=lengths)
+    case = prefill_case(gpu, lengths, heads=heads, seed=heads[1], dt_dtype=torch.bfloat16,
+                        w_dtype=torch.bfloat16)
+    case["has_initial"][1::2] = False
+    case["slots"][6] = -1
+    check(case)
+
+
+@pytest.mark.parametrize("lengths", [[64], [65], [64, 64, 64, 64], [65, 64, 64, 64],
+                                     [80, 33, 70, 81, 90]])
+def test_both_sides_of_the_rule(gpu, lengths):
+    """One prompt of 64 and of 65 tokens, four sequences of 64 on average and just above (128
+    pairs), five sequences (160 pairs)."""
+    announce(test="heads_rule", lengths=lengths)
+    check(prefill_case(gpu, lengths, seed=len(lengths)))
+
+
+@pytest.mark.parametrize("what", ["qkv", "gate", "out"])
+def test_unaligned_rows_give_the_aligned_bits(gpu, what):
+    announce(test="heads_unaligned", what=what)
+    case = prefill_case(gpu, [70, 33, 1, 0, 64, 90], seed=3)
+    pool0 = case["pool"].clone()
+    run(case)
+    torch.cuda.synchronize()
+    ref_out, ref_pool = case["out"].clone(), case["pool"].clone()
+    n = case["qkv"].shape[0]
+    if what == "out":
+        flat = torch.zeros(n * 32 * 128 + 1, dtype=torch.bfloat16, device=gpu)
+        case["out"] = flat[1:].view(n, 32, 128)
+    else:
+        rows = case[what].reshape(n, -1)
+        moved = torch.empty(n, rows.shape[1] + 3, dtype=torch.bfloat16, device=gpu)[:, 1:-2]
+        moved.copy_(rows)
+        case[what] = moved if what == "qkv" else moved.unflatten(1, (32, 128))
+    case["pool"].copy_(pool0)
+    run(case)
+    torch.cuda.synchronize()
+    assert torch.equal(case["out"], ref_out)
+    assert torch.equal(case["pool"], ref_pool)
+
+
+def test_rows_of_one_shared_token(gpu):
+    """qkv and gate as one row expanded over the tokens (row stride 0)."""
+    announce(test="heads_expanded_rows")
+    case = prefill_case(gpu, [40] * 6, seed=4)
+    n = case["qkv"].shape[0]
+    case["qkv"] = case["qkv"][:1].expand(n, -1)
+    case["gate"] = case["gate"][:1].expand(n, -1, -1)
+    check(case)
