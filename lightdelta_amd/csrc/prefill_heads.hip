@@ -24,17 +24,16 @@
 // gated RMSNorm of whole rows.  q, k and v come from qkv through LDS, the transposed operands
 // by ds_read_b64_tr_b16; T, P (as planes) and the per-token scales from the prep's records.
 //
-// What bounds it: the matrix pipe and the vector work of the splits.  A wave's chunk is 96
-// matrix instructions (3,072 cycles) and, with the norm, 690 vector ones, of which the 192
-// v_dot2 run alone (8 of them behind a matrix instruction took 78 cycles, 8 multiply-adds 43,
-// 6 of those 34), so about 4,200 cycles; two workgroups a CU take 4,800 per head and chunk.  At
-// 32 x 1024 tokens and 32 v-heads that is 0.94 PFLOP/s of bf16 products at a clock that the
-// card's power limit holds at 1.6 GHz (a large bf16 GEMM reaches 1.17), 438 us, where
-// chunk_scan32_kernel and the norm pass took 820 us: with a head's rows over four workgroups
-// every wave re-read S's planes from LDS and the raw outputs crossed HBM twice more.  The whole
-// prefill went from 985 to 625 us there, 257 to 179 us at 8 x 1024, 1,710 to 1,310 us at
-// 1024 x 32.  Products and vector work are laid out by hand, slot by slot: as the compiler
-// scheduled the same code, 32 x 1024 took 685 us.
+// What bounds it: vector issue and power.  A wave's chunk is 96 matrix instructions (3,072
+// cycles) and, with the norm, 880 vector ones (3,900 cycles of issue with the matrix ones');
+// two workgroups a CU take 8,700 cycles for a chunk each.  At 32 x 1024 tokens and 32 v-heads
+// that is 0.94 PFLOP/s of bf16 products, at a clock that the card's power limit holds at 1.6
+// GHz (a large bf16 GEMM reaches 1.17), 438 us, where chunk_scan32_kernel and the norm pass
+// took 820 us: with a head's rows over four workgroups every wave re-read S's planes from LDS
+// and the raw outputs crossed HBM twice more.  The whole prefill went from 985 to 625 us
+// there, 257 to 178 us at 8 x 1024, 1,710 to 1,310 us at 1024 x 32.  Products and vector work
+// are laid out by hand, slot by slot: as the compiler scheduled the same code, 32 x 1024 took
+// 685 us.
 #include "chunk_common.h"
 
 namespace ld {
@@ -68,32 +67,11 @@ __device__ __forceinline__ void pin(T& x) {
   asm volatile("" : "+v"(x));
 }
 
-// r - s for a pair of values and its rounded bf16 pair, both for four pairs: each value plus
-// the dot product of the pair with (-1, 0) or (0, -1), exact as in split4, but with the
-// three-operand form, which leaves r in place (the builtin's two-operand form costs a move per
-// value that lives on, as the state does).  The dots' results are ready for any instruction
-// three issue slots later: the block ends with the wait.
-__device__ __forceinline__ void remainders(const float (&r)[8], u32x4 w, float (&out)[8]) {
-  const uint32_t w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
-  asm volatile(
-      "v_dot2_f32_bf16 %0, %16, %20, %8\n\t"
-      "v_dot2_f32_bf16 %1, %16, %21, %9\n\t"
-      "v_dot2_f32_bf16 %2, %17, %20, %10\n\t"
-      "v_dot2_f32_bf16 %3, %17, %21, %11\n\t"
-      "v_dot2_f32_bf16 %4, %18, %20, %12\n\t"
-      "v_dot2_f32_bf16 %5, %18, %21, %13\n\t"
-      "v_dot2_f32_bf16 %6, %19, %20, %14\n\t"
-      "v_dot2_f32_bf16 %7, %19, %21, %15\n\t"
-      "s_nop 2"
-      : "=&v"(out[0]), "=&v"(out[1]), "=&v"(out[2]), "=&v"(out[3]), "=&v"(out[4]), "=&v"(out[5]),
-        "=&v"(out[6]), "=&v"(out[7])
-      : "v"(r[0]), "v"(r[1]), "v"(r[2]), "v"(r[3]), "v"(r[4]), "v"(r[5]), "v"(r[6]), "v"(r[7]),
-        "v"(w0), "v"(w1), "v"(w2), "v"(w3), "s"(0x0000bf80u), "s"(0xbf800000u));
-}
-
 // The exact split of eight values (a lane's registers 8 u .. 8 u + 7 of an accumulator) into
-// planes that are B operands, in five stages of 4 or 8 instructions: a stage fits beside one
-// matrix instruction.
+// planes that are B operands, in five stages: 0, 2, 4 round (4 instructions), 1, 3 take the
+// remainders (16: each value less its plane's, exact).  split4's remainder is one v_dot2c, but
+// that does not run beside a matrix instruction: with 8 of them behind each, a matrix
+// instruction of 32 cycles took 81 (78 with two waves a SIMD); with 8 of these, 46 (42).
 struct Split8 {
   float r[8];
   u32x4 w[3];
@@ -106,10 +84,14 @@ struct Split8 {
   }
   __device__ __forceinline__ void stage(int i) {  // 0 .. 4
     if (i & 1) {
-      float rest[8];
-      remainders(r, w[i >> 1], rest);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = rest[e];
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t pair = w[i >> 1][j];
+        r[2 * j] -= __builtin_bit_cast(float, pair << 16);
+        r[2 * j + 1] -= __builtin_bit_cast(float, pair & 0xffff0000u);
+      }
+      asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]),
+                   "+v"(r[6]), "+v"(r[7]));
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) w[i >> 1][j] = bf16_pair(f32x2{r[2 * j], r[2 * j + 1]});
@@ -169,55 +151,96 @@ __device__ __forceinline__ u32x4 load_piece(__amdgpu_buffer_rsrc_t rs, uint32_t 
 }
 
 // The gated RMSNorm of a chunk's rows, a thread's 16 columns of one token, in slices that fit
-// beside matrix instructions: 0: the raw outputs' reads, 1-4: squares, 5: the row's sum over its
-// 8 threads, 6: rstd, 7-22: two per pair of columns.  Arithmetic as prefill_norm_kernel's.
+// beside matrix instructions and hold eight independent operations where the arithmetic
+// allows: 0: the raw outputs' reads, 1-4: squares, 5: the row's sum over its 8 threads, 6:
+// rstd, 7-14: columns 0 .. 7, 15-22: columns 8 .. 15.  Arithmetic as prefill_norm_kernel's.
 struct Norm {
   u32x4 raw[2], gate[2], y[2];
-  float ss, rstd, sig0, sig1;
-  f32x2 w;
+  float ss[2], rstd, g[8], t[8];
+  __device__ __forceinline__ static float low(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
+  __device__ __forceinline__ static float high(uint32_t pair) {
+    return __builtin_bit_cast(float, pair & 0xffff0000u);
+  }
+  __device__ __forceinline__ void pin8(float (&x)[8]) {
+    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]),
+                 "+v"(x[6]), "+v"(x[7]));
+  }
   __device__ __forceinline__ void slice(int i, const uint8_t* raw0, const uint8_t* raw1,
                                         const float* weight, float eps) {
     if (i == 0) {
       raw[0] = *reinterpret_cast<const u32x4*>(raw0);
       raw[1] = *reinterpret_cast<const u32x4*>(raw1);
-      ss = 0.0f;
+      ss[0] = ss[1] = 0.0f;
     } else if (i < 5) {
 #pragma unroll
-      for (int d = 2 * ((i - 1) & 1); d < 2 * ((i - 1) & 1) + 2; ++d) {
-        const uint32_t bits = raw[(i - 1) >> 1][d];
-        const float lo = __builtin_bit_cast(float, bits << 16);
-        const float hi = __builtin_bit_cast(float, bits & 0xffff0000u);
-        ss = fmaf(lo, lo, ss);
-        ss = fmaf(hi, hi, ss);
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t bits = raw[h][i - 1];
+        ss[h] = fmaf(low(bits), low(bits), ss[h]);
+        ss[h] = fmaf(high(bits), high(bits), ss[h]);
       }
-      pin(ss);
+      pin(ss[0]);
+      pin(ss[1]);
     } else if (i == 5) {
-      ss += dpp<kDppQuadXor1>(ss);
-      ss += dpp<kDppQuadXor2>(ss);
-      ss += dpp<kDppRowHalfMirror>(ss);
-      pin(ss);
+      ss[0] += ss[1];
+      ss[0] += dpp<kDppQuadXor1>(ss[0]);
+      ss[0] += dpp<kDppQuadXor2>(ss[0]);
+      ss[0] += dpp<kDppRowHalfMirror>(ss[0]);
+      pin(ss[0]);
     } else if (i == 6) {
-      rstd = fast_rsqrt(ss / static_cast<float>(kDim) + eps);
+      rstd = fast_rsqrt(ss[0] / static_cast<float>(kDim) + eps);
       pin(rstd);
     } else {
-      const int j = (i - 7) >> 1;   // pair of columns
-      const uint32_t gb = gate[j >> 2][j & 3];
-      const float g0 = __builtin_bit_cast(float, gb << 16);
-      const float g1 = __builtin_bit_cast(float, gb & 0xffff0000u);
-      if ((i - 7) % 2 == 0) {
-        w = *reinterpret_cast<const f32x2*>(weight + 2 * j);
-        sig0 = sigmoid(g0);
-        sig1 = sigmoid(g1);
-        pin(sig0);
-        pin(sig1);
-      } else {
-        const uint32_t rb = raw[j >> 2][j & 3];
-        const float y0 =
-            ((__builtin_bit_cast(float, rb << 16) * rstd) * w.x) * (g0 * sig0);
-        const float y1 =
-            ((__builtin_bit_cast(float, rb & 0xffff0000u) * rstd) * w.y) * (g1 * sig1);
-        y[j >> 2][j & 3] = bf16_pair(f32x2{y0, y1});
-        pin(y[j >> 2]);
+      const int h = (i - 7) >> 3;
+      switch ((i - 7) & 7) {
+        case 0:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t pair = gate[h][e >> 1];
+            g[e] = e & 1 ? high(pair) : low(pair);
+          }
+          pin8(g);
+          break;
+        case 1:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] = __expf(-g[e]);
+          pin8(t);
+          break;
+        case 2:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] += 1.0f;
+          pin8(t);
+          break;
+        case 3:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] = fast_rcp(t[e]);
+          pin8(t);
+          break;
+        case 4:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] *= g[e];   // silu
+          pin8(t);
+          break;
+        case 5:
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t pair = raw[h][e >> 1];
+            g[e] = (e & 1 ? high(pair) : low(pair)) * rstd;
+          }
+          pin8(g);
+          break;
+        case 6: {
+          const f32x4 w0 = *reinterpret_cast<const f32x4*>(weight + 8 * h);
+          const f32x4 w1 = *reinterpret_cast<const f32x4*>(weight + 8 * h + 4);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) g[e] *= e < 4 ? w0[e & 3] : w1[e & 3];
+          pin8(g);
+          break;
+        }
+        default:
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            y[h][d] = bf16_pair(f32x2{g[2 * d] * t[2 * d], g[2 * d + 1] * t[2 * d + 1]});
+          pin(y[h]);
       }
     }
   }
@@ -257,7 +280,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   // columns of both); two, as the norm reads one while the next chunk's v arrives
   __shared__ __attribute__((aligned(16))) uint8_t sV[2][kTileSize];
   __shared__ __attribute__((aligned(16))) uint8_t sRec[R::kBytes];
-  __shared__ float sW[kDim];
+  __shared__ __attribute__((aligned(16))) float sW[kDim];
 
   if (tid < kDim) sW[tid] = load_param(p.norm_weight, tid, WBf16);
 
@@ -561,12 +584,19 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     for (int q = 0; q < 2; ++q) ck[q] = scales[R::kCk + 2 * q];
     // beside P X: the split of ck V_new (now: step 0, last: step 1)
     Split8 last;
+    auto scaled_vn = [&](int q, Split8& to) __attribute__((always_inline)) {
+      f32x4 lo = quad(vn, q) * ck[q];
+      f32x4 hi = quad(vn, q + 1) * ck[q + 1];
+      pin(lo);   // rounded: the first remainder is of the product's fp32 value
+      pin(hi);
+      to.set(lo, hi);
+    };
     auto slot_p0 = [&](int i) __attribute__((always_inline)) {
       if (i % 3 == 0) prefetch(6 + i / 3);
       if (i == 0) {
         normalise(4);
       } else if (i == 1) {
-        now.set(quad(vn, 0) * ck[0], quad(vn, 1) * ck[1]);
+        scaled_vn(0, now);
         now.stage(0);
       } else {
         now.stage(i - 1);
@@ -577,7 +607,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     auto slot_p1 = [&](int i) __attribute__((always_inline)) {
       if (i % 3 == 0) prefetch(8 + i / 3);
       if (i == 0)
-        last.set(quad(vn, 2) * ck[2], quad(vn, 3) * ck[3]);
+        scaled_vn(2, last);
       else
         last.stage(i - 1);
     };
