@@ -1,5 +1,6 @@
 // Device helpers shared by the chunked-prefill kernels (prefill_chunked.hip,
-// prefill_heads.hip): the exact three-way bf16 split of fp32 values and buffer-resource loads.
+// prefill_heads.hip): the exact three-way bf16 split of fp32 values, buffer-resource loads and
+// the chunk search.
 #pragma once
 
 #include "gdn_common.h"
@@ -95,6 +96,40 @@ __device__ __forceinline__ u32x4 load16u(__amdgpu_buffer_rsrc_t rsrc, uint32_t l
 
 __device__ __forceinline__ float load4(__amdgpu_buffer_rsrc_t rsrc, int byte_offset) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, 0, byte_offset, 0));
+}
+
+// Global chunk g -> (sequence, first row, tokens): the last n with chunk_start[n] <= g
+// (empty sequences come before it), by a 64-way search with one wave-wide load per level
+// (one level up to 64 sequences, two up to 4096; a binary search took one dependent load per
+// halving); false past the last chunk.  Called by every lane of a wave; the results are
+// uniform.  C: tokens per chunk.
+template <int C>
+__device__ bool find_chunk(const int32_t* cu, const int32_t* chunk_start, int num_sequences,
+                           int g, int& seq, int& t0, int& len) {
+  if (g >= chunk_start[num_sequences]) return false;
+  const int lane = threadIdx.x & 63;
+  int lo = 0;              // chunk_start[lo] <= g throughout
+  int count = num_sequences;
+  for (;;) {
+    const int step = (count + 63) >> 6;   // entries per lane at this level
+    const bool in = lane * step < count;
+    const int idx = lo + (in ? lane * step : 0);
+    const int start = chunk_start[idx];
+    int row0 = 0, row1 = 0;
+    if (step == 1) {   // the last level: the rows of every candidate in the same round trip
+      row0 = cu[idx];
+      row1 = cu[idx + 1];
+    }
+    const int k = 63 - __clzll(static_cast<long long>(__ballot(in && start <= g)));
+    if (step == 1) {
+      seq = lo + k;
+      t0 = __builtin_amdgcn_readlane(row0, k) + (g - __builtin_amdgcn_readlane(start, k)) * C;
+      len = min(C, __builtin_amdgcn_readlane(row1, k) - t0);
+      return true;
+    }
+    lo += k * step;
+    count = min(step, count - k * step);
+  }
 }
 
 }  // namespace

@@ -138,40 +138,6 @@ __global__ __launch_bounds__(kThreads) void chunk_index_kernel(const int32_t* cu
   }
 }
 
-// Global chunk g -> (sequence, first row, tokens): the last n with chunk_start[n] <= g
-// (empty sequences come before it), by a 64-way search with one wave-wide load per level
-// (one level up to 64 sequences, two up to 4096; a binary search took one dependent load per
-// halving); false past the last chunk.  Called by every lane of a wave; the results are
-// uniform.  C: tokens per chunk.
-template <int C>
-__device__ bool find_chunk(const int32_t* cu, const int32_t* chunk_start, int num_sequences,
-                           int g, int& seq, int& t0, int& len) {
-  if (g >= chunk_start[num_sequences]) return false;
-  const int lane = threadIdx.x & 63;
-  int lo = 0;              // chunk_start[lo] <= g throughout
-  int count = num_sequences;
-  for (;;) {
-    const int step = (count + 63) >> 6;   // entries per lane at this level
-    const bool in = lane * step < count;
-    const int idx = lo + (in ? lane * step : 0);
-    const int start = chunk_start[idx];
-    int row0 = 0, row1 = 0;
-    if (step == 1) {   // the last level: the rows of every candidate in the same round trip
-      row0 = cu[idx];
-      row1 = cu[idx + 1];
-    }
-    const int k = 63 - __clzll(static_cast<long long>(__ballot(in && start <= g)));
-    if (step == 1) {
-      seq = lo + k;
-      t0 = __builtin_amdgcn_readlane(row0, k) + (g - __builtin_amdgcn_readlane(start, k)) * C;
-      len = min(C, __builtin_amdgcn_readlane(row1, k) - t0);
-      return true;
-    }
-    lo += k * step;
-    count = min(step, count - k * step);
-  }
-}
-
 // The 20 tiles of A (K K^T) and P (Q K^T) on or below the diagonal over the prep's 8 waves:
 // 3 each for waves 0-3 and 2 each for waves 4-7 (so 5 per SIMD, waves w and w + 4 sharing
 // one), 5 bits a tile, (is_p << 4) | (row tile << 2) | column tile.
@@ -687,16 +653,6 @@ __device__ __forceinline__ int piece32(int mt, int nt, int lg, int li) {
   return ((mt * 2 + (lg & 1)) * 64 + (2 * nt + (lg >> 1)) * 16 + li) * 4;
 }
 
-// Columns j .. j + 3 (j a multiple of 4) of row i of a 32 x 32 matrix into its planes in a
-// HeadRecord (byte offset `base`).
-__device__ __forceinline__ void put_planes(float* rec, int base, int i, int j, f32x4 x) {
-  const Split4 sp = split4(x);
-  uint8_t* at = reinterpret_cast<uint8_t*>(rec) + base + (j >> 4) * 3072 +
-                (((j >> 2) & 1) * 32 + i) * 16 + ((j >> 3) & 1) * 8;
-#pragma unroll
-  for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint2*>(at + pl * 1024) = sp.p[pl];
-}
-
 // The 6 tiles of A (K K^T) and P (Q K^T) on or below the diagonal, as tile_code: A00, A10,
 // A11, P00, P10, P11; wave w takes tiles w and w + 4.
 __device__ __forceinline__ uint32_t prep32_tile(int index) {
@@ -710,14 +666,13 @@ __device__ __forceinline__ uint32_t prep32_tile(int index) {
   }
 }
 
-template <bool DtBf16, bool Wide, bool Heads>
+template <bool DtBf16, bool Wide>
 __global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
 void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
                          const int32_t* chunk_start, int records) {
   using R = Rec32;
   constexpr int kCs = R::kC;
   constexpr int kTokens = kCs / (kPrep32Threads / 64);   // tokens normalised per wave
-  constexpr int64_t kRec = Heads ? HeadRecord::kBytes / 4 : R::kSize;   // floats
   const int64_t unit = blockIdx.x;   // chunk * H + k-head
   const int g = static_cast<int>(unit / p.num_k_heads);
   if (g >= records) return;
@@ -739,12 +694,9 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
   __shared__ __attribute__((aligned(16))) uint16_t sKh[kCs][kHRow];
   __shared__ __attribute__((aligned(16))) float sA[kCs][kARow];     // -A of the v-head
   __shared__ __attribute__((aligned(16))) float sT[3][16][kTRow];   // T0, T1, T10
-  // Heads: P0 of the v-head, double-buffered (the next v-head's is written while waves still
-  // multiply this one's)
-  __shared__ __attribute__((aligned(16))) float sP[Heads ? 2 : 1][Heads ? kCs : 1][kARow];
   // a v-head's gates, double-buffered (v-head m in buffer m & 1): G_i, beta_i, exp(G_i),
   // exp(G_n-1 - G_i), one entry per lane of the wave that forms them
-  __shared__ __attribute__((aligned(16))) float sGates[2][4][64];
+  __shared__ float sGates[2][4][64];
   __shared__ float sRq[kCs];   // rq_i scale (zero past the end)
   __shared__ float sRk[kCs];   // rk_i (zero past the end)
 
@@ -779,8 +731,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
     gb[2][lane] = __expf(G);
     gb[3][lane] = __expf(glast - G);
     if (lane == 0)
-      ws[(static_cast<int64_t>(g) * p.num_v_heads + head) * kRec +
-         (Heads ? HeadRecord::kGamma / 4 : R::kOffMisc)] = __expf(glast);
+      ws[(static_cast<int64_t>(g) * p.num_v_heads + head) * R::kSize + R::kOffMisc] = __expf(glast);
   };
   if (wave == 3) fetch_gates(key_head * p.group);
 
@@ -860,7 +811,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
 
   // Qr, Kq and Kr (the bf16 inputs in the scan's load order, item = one 16-byte piece) to
   // the record of the group's first v-head
-  if constexpr (!Heads) {
+  {
     float* rec0 = ws + (static_cast<int64_t>(g) * p.num_v_heads + key_head * p.group) * R::kSize;
     u32x4* qdst = reinterpret_cast<u32x4*>(rec0 + R::kOffQr);
     u32x4* kqdst = reinterpret_cast<u32x4*>(rec0 + R::kOffKq);
@@ -910,7 +861,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
   for (int member = 0; member < p.group; ++member) {
     const int head = key_head * p.group + member;
     const bool next = member + 1 < p.group;
-    float* rec = ws + (static_cast<int64_t>(g) * p.num_v_heads + head) * kRec;
+    float* rec = ws + (static_cast<int64_t>(g) * p.num_v_heads + head) * R::kSize;
     const float* const sG = sGates[member & 1][0];
     const float* const sBeta = sGates[member & 1][1];
     const float* const sEg = sGates[member & 1][2];
@@ -918,16 +869,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
 
     // the per-token scales: sq = rq scale exp(G), beta, ck = rk exp(G_n-1 - G),
     // ws = beta exp(G) rk (the 64-token prep's W scale)
-    if constexpr (Heads) {   // without beta, which is in T's columns
-      constexpr int kAt = HeadRecord::kScales / 4;
-      if (tid < kCs) {
-        rec[kAt + 4 * HeadRecord::kSq + tid] = sRq[tid] * sEg[tid];
-        rec[kAt + 4 * HeadRecord::kWs + tid] = sEg[tid] * sRk[tid];
-      } else if (tid < 2 * kCs) {
-        const int j = tid - kCs;
-        rec[kAt + 4 * HeadRecord::kCk + j] = sRk[j] * sEk[j];
-      }
-    } else if (tid < kCs) {
+    if (tid < kCs) {
       rec[R::kOffMisc + kMiscSq + tid] = sRq[tid] * sEg[tid];
       rec[R::kOffMisc + kMiscBeta + tid] = sBeta[tid];
     } else if (tid < 2 * kCs) {
@@ -956,10 +898,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
           const float gam = __expf(gi - sG[m]);
           piece[r] = (m <= i && i < len) ? gam * ((rqi * sRk[m]) * prod[t][r]) : 0.0f;
         }
-        if constexpr (Heads)
-          *reinterpret_cast<f32x4*>(&sP[member & 1][i][16 * nt + 4 * lg]) = piece;
-        else
-          *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(mt, nt, lg, li)) = piece;
+        *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(mt, nt, lg, li)) = piece;
       } else {
         const int m = 16 * nt + li;
         const float gm = sG[m];
@@ -972,11 +911,9 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
         }
       }
     }
-    if constexpr (!Heads) {
-      if (wave == 2)
-        *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(0, 1, lg, li)) =
-            f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    if (wave == 2)
+      *reinterpret_cast<f32x4*>(rec + R::kOffP + piece32(0, 1, lg, li)) =
+          f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     __syncthreads();   // -A complete
     if (wave == 3 && next) gates(member + 1);
     // inverses of the unit lower-triangular diagonal blocks (I + A_bb), column li per lane
@@ -1021,32 +958,7 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
       else
         v = c < 16 ? *reinterpret_cast<const f32x4*>(&sT[2][li][c])
                    : *reinterpret_cast<const f32x4*>(&sT[1][li][c - 16]);
-      if constexpr (Heads)
-        put_planes(rec, HeadRecord::kT, 16 * w + li, c, v * *reinterpret_cast<const f32x4*>(&sBeta[c]));
-      else
-        *reinterpret_cast<f32x4*>(rec + R::kOffT + tid * 4) = v;
-    }
-    // P = P0 T, transposed (T^T P0^T), so that a lane's four results are four consecutive
-    // columns of row li of a tile: blocks (0, 0), (1, 0), (1, 1) by waves 0, 1, 2, and the zero
-    // block by wave 3; the summation index k = 4 lg + step as above
-    if constexpr (Heads) {
-      f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (wave < 3) {
-        const int mt = wave > 0 ? 1 : 0;
-        const int nt = wave > 1 ? 1 : 0;
-        const f32x4 p0 = *reinterpret_cast<const f32x4*>(&sP[member & 1][16 * mt + li][16 * nt + 4 * lg]);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) d = mfma(sT[nt][4 * lg + st][li], p0[st], d);
-        if (wave == 1) {   // + P0 (1, 1) T10
-          const f32x4 p1 = *reinterpret_cast<const f32x4*>(&sP[member & 1][16 + li][16 + 4 * lg]);
-#pragma unroll
-          for (int st = 0; st < 4; ++st) d = mfma(sT[2][4 * lg + st][li], p1[st], d);
-        }
-        d *= *reinterpret_cast<const f32x4*>(&sBeta[16 * nt + 4 * lg]);
-        put_planes(rec, HeadRecord::kP, 16 * mt + li, 16 * nt + 4 * lg, d);
-      } else {
-        put_planes(rec, HeadRecord::kP, li, 16 + 4 * lg, d);
-      }
+      *reinterpret_cast<f32x4*>(rec + R::kOffT + tid * 4) = v;
     }
     // the next v-head writes -A after its first barrier (every read of -A and T above is
     // behind one of this v-head's) and its gates went to the other buffer
@@ -1852,7 +1764,7 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
 // the second's chain is the shorter; from two chunks per CU on the first's throughput decides,
 // and for prompts of one or two chunks the launch it saves (us, first / second, at 32 v-heads:
 // 1 x 64 27 / 28, 1 x 256 46 / 35, 4 x 256 50.9 / 49.8, 4 x 1024 144 / 137, 5 x 1024 150 / 181,
-// 8 x 128 41 / 50, 8 x 1024 179 / 258, 32 x 1024 625 / 985, 1024 x 32 1310 / 1710).
+// 8 x 128 41 / 50, 8 x 1024 164 / 258, 32 x 1024 586 / 985, 1024 x 32 1264 / 1710).
 bool whole_heads(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
   return num_sequences * num_v_heads > 128 || num_tokens <= 64 * num_sequences;
 }
@@ -1875,38 +1787,33 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   *normed = heads;
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;
-#define LD_PREP_LAUNCH(K, D, W, N, ...)                                                        \
-  hipLaunchKernelGGL((K<D, W __VA_OPT__(, ) __VA_ARGS__>), per_chunk, dim3(N), 0, stream, p, num_sequences, ws,          \
+#define LD_PREP_LAUNCH(K, D, W, N)                                                             \
+  hipLaunchKernelGGL((K<D, W>), per_chunk, dim3(N), 0, stream, p, num_sequences, ws,          \
                      chunk_start, static_cast<int>(chunks))
-#define LD_PREP_LAUNCHES(K, N, ...)                                                            \
+#define LD_PREP_LAUNCHES(K, N)                                                                 \
   if (dt_bf16) {                                                                               \
     if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, true, true, N, __VA_ARGS__);                                                        \
+      LD_PREP_LAUNCH(K, true, true, N);                                                        \
     else                                                                                       \
-      LD_PREP_LAUNCH(K, true, false, N, __VA_ARGS__);                                                       \
+      LD_PREP_LAUNCH(K, true, false, N);                                                       \
   } else {                                                                                     \
     if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, false, true, N, __VA_ARGS__);                                                       \
+      LD_PREP_LAUNCH(K, false, true, N);                                                       \
     else                                                                                       \
-      LD_PREP_LAUNCH(K, false, false, N, __VA_ARGS__);                                                      \
+      LD_PREP_LAUNCH(K, false, false, N);                                                      \
   }
+  if (heads)
+    return launch_chunk_heads(p, num_sequences, ws, chunk_start, static_cast<int>(chunks), dt_bf16,
+                              w_bf16, stream);
   if constexpr (TT == 2) {
-    if (heads) {
-      LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads, true)
-    } else {
-      LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads, false)
-    }
+    LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads)
   } else {
     LD_PREP_LAUNCHES(chunk_prep_kernel, kPrepThreads)
   }
 #undef LD_PREP_LAUNCHES
 #undef LD_PREP_LAUNCH
   const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
-  if (heads) {
-    const int rc = launch_chunk_heads(p, num_sequences, ws, chunk_start, static_cast<int>(chunks),
-                                      w_bf16, stream);
-    if (rc != LD_OK) return rc;
-  } else if constexpr (TT == 2) {
+  if constexpr (TT == 2) {
     const int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
     if (scan_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
     hipLaunchKernelGGL(chunk_scan32_kernel, dim3(static_cast<uint32_t>(scan_groups)),

@@ -30,8 +30,9 @@
 // that is 0.94 PFLOP/s of bf16 products, at a clock that the card's power limit holds at 1.6
 // GHz (a large bf16 GEMM reaches 1.17), 438 us, where chunk_scan32_kernel and the norm pass
 // took 820 us: with a head's rows over four workgroups every wave re-read S's planes from LDS
-// and the raw outputs crossed HBM twice more.  The whole prefill went from 985 to 625 us
-// there, 257 to 178 us at 8 x 1024, 1,710 to 1,310 us at 1024 x 32.  Products and vector work
+// and the raw outputs crossed HBM twice more.  The whole prefill, with the prep
+// below, went from 985 to 586 us there, 257 to 164 us at 8 x 1024, 1,710 to 1,264 us at
+// 1024 x 32.  Products and vector work
 // are laid out by hand, slot by slot: as the compiler scheduled the same code, 32 x 1024 took
 // 685 us.
 #include "chunk_common.h"
@@ -46,6 +47,10 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 constexpr int kTok = HeadRecord::kTokens;
 constexpr int kTileRow = kDim * 2;             // bytes of a q, k, v or raw-output row in LDS
 constexpr int kTileSize = kTok * kTileRow;
+// A chunk's record in LDS: T's and P's planes, plane i of step u at 3072 u + 1024 i, the scales.
+constexpr int kLdsT = 0;
+constexpr int kLdsP = 6144;
+constexpr int kLdsScales = 12288;
 
 // 16-byte pieces of row r are stored at piece ^ swizzle(r): a column of pieces over 16 rows
 // (operand A of the products with S) and 4 x 4 element blocks of 4 rows (transposed reads)
@@ -133,6 +138,10 @@ __device__ __forceinline__ bf16x4 read_tr(const uint8_t* at) {
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
+
+// Keeps LDS accesses of a wave in program order past the compiler (the hardware runs them in
+// order).
+__device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
 // Sixteen bytes of a row at a lane's byte offset + a uniform one: one load, or (rows not at
 // 16-byte boundaries) eight of one element.
@@ -246,6 +255,259 @@ struct Norm {
   }
 };
 
+// ---- the records: one wave per (chunk, k-head) ------------------------------------------
+// A wave does a whole unit alone, so nothing waits on another wave: q and k come as operands of
+// v_mfma_f32_16x16x32_bf16 (for lane l, li = l % 16 and lg = l / 16: row 16 a + li, 16 bytes at
+// k = 32 s + 8 lg), which give the raw products K K^T and K Q^T below the diagonal and, from
+// the diagonals of K K^T and Q Q^T, the squared norms; then each v-head of the group in turn:
+// gates, -A to LDS, the inverses of I + A's two diagonal blocks (a column per lane), T10 =
+// -T1 A10 T0 and P = P0 T as 16 x 16 x 4 fp32 products with summation index k = 4 lg + step,
+// for which P0's tiles, T10 and the first product are operands as they are.
+// Bound by memory and by the latency of its chain: at 32 x 1024 tokens, 32 v-heads, 113 us for
+// 0.59 GB, where a workgroup of four waves with a barrier per phase took 169 us (0.69 GB, with
+// the planes' zero rows); at 512 prompts of 8 to 56 tokens 80 us against 132.
+constexpr int kPrepWaves = 4;
+
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// c[4 lg + r][li] + sum over k of a[li][k] b[k][li], the lane's a[li][4 lg + st] and
+// b[4 lg + st][li]
+__device__ __forceinline__ f32x4 mfma_f32(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int st = 0; st < 4; ++st) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], b[st], c, 0, 0, 0);
+  return c;
+}
+
+// Inclusive sums over the 32 lanes of each half wave (lane 32 + i as lane i).
+__device__ __forceinline__ float prefix_sum32(float x, int lane) {
+  x += dpp<0x111>(x);   // row_shr:1, 2, 4, 8: zeros from below the row
+  x += dpp<0x112>(x);
+  x += dpp<0x114>(x);
+  x += dpp<0x118>(x);
+  const float row0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 15));
+  return x + ((lane & 16) != 0 ? row0 : 0.0f);
+}
+
+template <bool DtBf16, bool Wide>
+__global__ __launch_bounds__(64 * kPrepWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
+                             const int32_t* chunk_start, int records) {
+  using R = HeadRecord;
+  constexpr int kARow = kTok + 4;   // padded rows (floats)
+  constexpr int kTRow = 20;
+  struct Scratch {
+    float a[kTok][kARow];           // -A
+    float t[3][16][kTRow];          // T0, T1, T10
+    float g[kTok], beta[kTok], rq[kTok], rk[kTok];
+  };
+  __shared__ __attribute__((aligned(16))) Scratch scratch[kPrepWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  Scratch& sc = scratch[wave];
+  const int64_t unit = static_cast<int64_t>(blockIdx.x) * kPrepWaves + wave;   // chunk * H + k-head
+  const int g = static_cast<int>(unit / p.num_k_heads);
+  if (g >= records) return;
+  const int key_head = static_cast<int>(unit - static_cast<int64_t>(g) * p.num_k_heads);
+  int seq = 0, t0 = 0, len = 0;
+  if (!find_chunk<kTok>(p.cu, chunk_start, num_sequences, g, seq, t0, len)) return;
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+
+  // a v-head's gate inputs, lane = token (lanes 32 .. 63 as 0 .. 31), fetched one v-head ahead
+  const int token = lane & 31;
+  uint16_t gate_a = 0, gate_b = 0;
+  float gate_a_log = 0.0f, gate_dt_bias = 0.0f;
+  auto fetch_gates = [&](int head) __attribute__((always_inline)) {
+    const int64_t tok = t0 + min(token, len - 1);
+    gate_a = p.a[tok * p.a_row + head];
+    gate_b = p.b[tok * p.b_row + head];
+    gate_a_log = p.a_log[head];
+    gate_dt_bias = load_param(p.dt_bias, head, DtBf16);
+  };
+  fetch_gates(key_head * p.group);
+
+  // raw tiles of the inputs (exact products, fp32 sums): kk[0, 1, 2] = K K^T (0,0), (1,0), (1,1),
+  // rows 4 lg + r, column li; kq = K Q^T of P's tiles (0,0), (1,0), (1,1): row li of P0, columns
+  // 4 lg + r
+  f32x4 kk[3], kq[3];
+  {
+    const uint32_t row_bytes = static_cast<uint32_t>(p.qkv_row) * 2;
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.qkv + static_cast<int64_t>(t0) * p.qkv_row), 0,
+        (len - 1) * static_cast<int>(row_bytes) + (2 * p.num_k_heads + p.num_v_heads) * kTileRow,
+        0x00020000);
+    u32x4 q[2][4], k[2][4];   // zeros past the chunk's end
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const uint32_t at = 16 * a + li < len ? (16 * a + li) * row_bytes + lg * 16 : 0xfffff000u;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        k[a][s] = load_piece<Wide>(rows, at, (p.num_k_heads + key_head) * kTileRow + s * 64);
+        q[a][s] = load_piece<Wide>(rows, at, key_head * kTileRow + s * 64);
+      }
+    }
+    f32x4 qq[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) kk[i] = kq[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    qq[0] = qq[1] = kk[0];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bf16x8 k0 = __builtin_bit_cast(bf16x8, k[0][s]);
+      const bf16x8 k1 = __builtin_bit_cast(bf16x8, k[1][s]);
+      const bf16x8 q0 = __builtin_bit_cast(bf16x8, q[0][s]);
+      const bf16x8 q1 = __builtin_bit_cast(bf16x8, q[1][s]);
+      kk[0] = mfma16(k0, k0, kk[0]);
+      kk[1] = mfma16(k1, k0, kk[1]);
+      kk[2] = mfma16(k1, k1, kk[2]);
+      kq[0] = mfma16(k0, q0, kq[0]);
+      kq[1] = mfma16(k0, q1, kq[1]);
+      kq[2] = mfma16(k1, q1, kq[2]);
+      qq[0] = mfma16(q0, q0, qq[0]);
+      qq[1] = mfma16(q1, q1, qq[1]);
+    }
+    // the inverse norms, from the lanes that hold a diagonal entry (register li % 4 of the lanes
+    // with li / 4 = lg); rows past the end: q's are zeros, k's too
+    if ((li >> 2) == lg) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const f32x4 dq = qq[a];
+        const f32x4 dk = kk[2 * a];
+        const int r = li & 3;
+        const float q2 = r < 2 ? (r == 0 ? dq[0] : dq[1]) : (r == 2 ? dq[2] : dq[3]);
+        const float k2 = r < 2 ? (r == 0 ? dk[0] : dk[1]) : (r == 2 ? dk[2] : dk[3]);
+        const bool live = 16 * a + li < len;
+        sc.rq[16 * a + li] = live ? fast_rsqrt(q2 + 1e-6f) * p.scale : 0.0f;
+        sc.rk[16 * a + li] = live ? fast_rsqrt(k2 + 1e-6f) : 0.0f;
+      }
+    }
+  }
+  lds_order();
+
+  const auto at4 = [](const float* x) __attribute__((always_inline)) {
+    return *reinterpret_cast<const f32x4*>(x);
+  };
+  for (int member = 0; member < p.group; ++member) {
+    const int head = key_head * p.group + member;
+    uint8_t* const rec = reinterpret_cast<uint8_t*>(ws) +
+                         (static_cast<int64_t>(g) * p.num_v_heads + head) * R::kBytes;
+    // gates and the in-chunk cumulative log decay: the token-serial form's arithmetic
+    {
+      const bool live = token < len;
+      const float x = bf16_to_f32(gate_a) + gate_dt_bias;
+      const float gl = live ? -__expf(gate_a_log) * softplus(x) : 0.0f;
+      const float beta = live ? sigmoid(bf16_to_f32(gate_b)) : 0.0f;
+      if (member + 1 < p.group) fetch_gates(head + 1);
+      const float G = prefix_sum32(gl, lane);
+      const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(G), 31));
+      const float eg = __expf(G);
+      const float rk = sc.rk[token];
+      float* const scales = reinterpret_cast<float*>(rec + R::kScales);
+      if (lane < kTok) {
+        sc.g[token] = G;
+        sc.beta[token] = beta;
+        scales[4 * R::kSq + token] = sc.rq[token] * eg;
+        scales[4 * R::kWs + token] = eg * rk;
+      } else {
+        scales[4 * R::kCk + token] = rk * __expf(glast - G);
+        if (token == 0) *reinterpret_cast<float*>(rec + R::kGamma) = __expf(glast);
+      }
+    }
+    lds_order();
+
+    // -A to LDS (tile i, rows 4 lg + r, column li), zeros from the diagonal on
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int mt = i > 0 ? 1 : 0, nt = i > 1 ? 1 : 0;
+      const int mcol = 16 * nt + li;
+      const float gm = sc.g[mcol];
+      const float rkm = sc.rk[mcol];
+      const f32x4 gi = at4(&sc.g[16 * mt + 4 * lg]);
+      const f32x4 bi = at4(&sc.beta[16 * mt + 4 * lg]);
+      const f32x4 rki = at4(&sc.rk[16 * mt + 4 * lg]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = -(bi[r] * __expf(gi[r] - gm) * ((rki[r] * rkm) * kk[i][r]));
+        sc.a[16 * mt + 4 * lg + r][mcol] = i == 1 || li < 4 * lg + r ? x : 0.0f;
+      }
+    }
+    // P0's tiles: row li, columns 4 lg + r
+    f32x4 p0[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int mt = i > 0 ? 1 : 0, nt = i > 1 ? 1 : 0;
+      const float gi = sc.g[16 * mt + li];
+      const float rqi = sc.rq[16 * mt + li];
+      const f32x4 gm = at4(&sc.g[16 * nt + 4 * lg]);
+      const f32x4 rkm = at4(&sc.rk[16 * nt + 4 * lg]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = __expf(gi - gm[r]) * ((rqi * rkm[r]) * kq[i][r]);
+        p0[i][r] = (i == 1 || 4 * lg + r <= li) && 16 * mt + li < len ? x : 0.0f;
+      }
+    }
+    lds_order();
+    // T0 and T1: column li of block lane / 16 (lanes 32 .. 63 repeat), row by row: col[i] =
+    // delta(i, li) + sum over m < i of (-A)[i][m] col[m], the terms in order of m
+    {
+      const int block = (lane >> 4) & 1;
+      const float* const ab = &sc.a[16 * block][16 * block];
+      float col[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) col[i] = i == li ? 1.0f : 0.0f;
+#pragma unroll
+      for (int mc = 0; mc < 15; ++mc)
+#pragma unroll
+        for (int i = mc + 1; i < 16; ++i) col[i] = fmaf(ab[i * kARow + mc], col[mc], col[i]);
+      if (lane < 32) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc.t[block][i][li] = col[i];
+      }
+    }
+    lds_order();
+    f32x4 t0k, t1k;   // T0, T1 [4 lg + r][li]
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      t0k[r] = sc.t[0][4 * lg + r][li];
+      t1k[r] = sc.t[1][4 * lg + r][li];
+    }
+    const f32x4 t0r = at4(&sc.t[0][li][4 * lg]);   // T0, T1 [li][4 lg + r]
+    const f32x4 t1r = at4(&sc.t[1][li][4 * lg]);
+    const f32x4 a10 = at4(&sc.a[16 + li][4 * lg]);
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const f32x4 z = mfma_f32(a10, t0k, zero);      // -A10 T0
+    const f32x4 t10k = mfma_f32(t1r, z, zero);     // T10 [4 lg + r][li]
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sc.t[2][4 * lg + r][li] = t10k[r];
+    // P = P0 T, transposed (T^T P0^T): row li, columns 4 lg + r
+    f32x4 pt[3];
+    pt[0] = mfma_f32(t0k, p0[0], zero);
+    pt[1] = mfma_f32(t10k, p0[2], mfma_f32(t0k, p0[1], zero));
+    pt[2] = mfma_f32(t1k, p0[2], zero);
+    lds_order();
+    const f32x4 t10r = at4(&sc.t[2][li][4 * lg]);
+    const f32x4 b0 = at4(&sc.beta[4 * lg]);
+    const f32x4 b1 = at4(&sc.beta[16 + 4 * lg]);
+    // to the planes: tile (mt, nt), row li, columns 4 lg ..
+    auto put = [&](int base, int mt, int nt, f32x4 x) __attribute__((always_inline)) {
+      const Split4 sp = split4(x);
+      uint8_t* const at = rec + base + (lg >> 1) * 8 + li * 16 +
+                          (nt == 0 ? (lg & 1) * 512 + mt * 256 : 3072 + (lg & 1) * 256);
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl)
+        *reinterpret_cast<uint2*>(at + pl * (nt == 0 ? 1024 : 512)) = sp.p[pl];
+    };
+    put(R::kT, 0, 0, t0r * b0);
+    put(R::kT, 1, 0, t10r * b0);
+    put(R::kT, 1, 1, t1r * b1);
+    put(R::kP, 0, 0, pt[0] * b0);
+    put(R::kP, 1, 0, pt[1] * b0);
+    put(R::kP, 1, 1, pt[2] * b1);
+    lds_order();   // (the next v-head rewrites the scratch)
+  }
+}
+
 // Wide: the rows of qkv, gate and out start at 16-byte boundaries.
 template <bool WBf16, bool Wide>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -279,7 +541,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   // v of the chunk, then in its place the raw outputs (a wave reads and writes its own 32
   // columns of both); two, as the norm reads one while the next chunk's v arrives
   __shared__ __attribute__((aligned(16))) uint8_t sV[2][kTileSize];
-  __shared__ __attribute__((aligned(16))) uint8_t sRec[R::kBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t sRec[kLdsScales + R::kBytes - R::kScales];
   __shared__ __attribute__((aligned(16))) float sW[kDim];
 
   if (tid < kDim) sW[tid] = load_param(p.norm_weight, tid, WBf16);
@@ -294,9 +556,23 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   const int v_col = (2 * p.num_k_heads + head) * kTileRow;
   const int qkv_bytes = (2 * p.num_k_heads + p.num_v_heads) * kTileRow;
   const uint32_t dst = srow * kTileRow + ((spiece ^ swizzle(srow)) << 4);
+  // where the record's bytes go in LDS: both steps' planes whole there (1024 bytes each), step
+  // 1's upper rows zeroed once
+  auto lds_at = [](int byte) __attribute__((always_inline)) {
+    const int base = byte < R::kP ? 0 : kLdsP;
+    const int at = byte < R::kP ? byte : byte - R::kP;
+    const int step1 = at - 3072;
+    return base + (at < 3072 ? at
+                             : 3072 + (step1 >> 9) * 1024 + ((step1 >> 8) & 1) * 512 + 256 + (step1 & 255));
+  };
+  const int rec_at[2] = {lds_at(tid * 16), lds_at(4096 + tid * 16)};
+  const int rest_at = lds_at(8192 + tid * 4);
+  for (int i = tid; i < 2 * 3 * 2 * 16; i += kThreads)   // matrix, plane, hi, 16-byte piece
+    *reinterpret_cast<u32x4*>(sRec + (i / 96) * kLdsP + 3072 + ((i / 32) % 3) * 1024 +
+                              ((i >> 4) & 1) * 512 + (i & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
   struct Staged {
-    u32x4 q[2], k[2], v[2], rec[3];
-    uint32_t scales;
+    u32x4 q[2], k[2], v[2], rec[2];
+    uint32_t rest, scales;   // the planes' last KiB and the scales, a word per thread
   };
   // Where chunk c's operands are (past the last chunk: resources over 0 bytes, whose loads
   // return zeros), and its load i of 10.
@@ -327,8 +603,10 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       x.q[i - 2] = load_piece<Wide>(from.rows, from.at[i - 2], q_col);
     else if (i < 6)
       x.v[i - 4] = load_piece<Wide>(from.rows, from.at[i - 4], v_col);
-    else if (i < 9)
+    else if (i < 8)
       x.rec[i - 6] = load16u(from.rec, tid * 16 + (i - 6) * 4096, 0);
+    else if (i == 8)
+      x.rest = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + 8192, 0, 0);
     else
       x.scales = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + R::kScales, 0, 0);
   };
@@ -340,12 +618,13 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       *reinterpret_cast<u32x4*>(sV[buf] + dst + i * 16 * kTileRow) = x.v[i];
     }
 #pragma unroll
-    for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(sRec + tid * 16 + i * 4096) = x.rec[i];
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sRec + rec_at[i]) = x.rec[i];
+    *reinterpret_cast<uint32_t*>(sRec + rest_at) = x.rest;
     if (tid < (R::kBytes - R::kScales) / 4)
-      *reinterpret_cast<uint32_t*>(sRec + tid * 4 + R::kScales) = x.scales;
+      *reinterpret_cast<uint32_t*>(sRec + kLdsScales + tid * 4) = x.scales;
   };
-  static_assert(R::kScales == 3 * 4096 && R::kBytes - R::kScales <= kThreads * 4,
-                "three pieces and a scale per thread");
+  static_assert(R::kScales == 2 * 4096 + 1024 && R::kBytes - R::kScales <= kThreads * 4,
+                "two pieces, a word and a scale per thread");
 
   Staged staged;
   if (chunks > 0) {
@@ -384,7 +663,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   const uint32_t raw_at =
       4 * hi * kTileRow + (((4 * w + (lj >> 3)) ^ hi) << 4) + (lj & 7) * 2;
   const uint8_t* const planes = sRec + lane * 16;
-  const f32x4* const scales = reinterpret_cast<const f32x4*>(sRec + R::kScales) + hi;
+  const f32x4* const scales = reinterpret_cast<const f32x4*>(sRec + kLdsScales) + hi;
 
   // The norm of chunk c - 1 runs beside chunk c's products; thread = (token, 16 columns).
   // Resources over the chunk's rows of gate and out (before the first chunk: over 0 bytes,
@@ -456,7 +735,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     auto operand = [&](const uint8_t* tile, int n) __attribute__((always_inline)) {
       return *reinterpret_cast<const bf16x8*>(tile + (a_at ^ (n << 5)));
     };
-    const float gamma = *reinterpret_cast<const float*>(sRec + R::kGamma);
+    const float gamma = *reinterpret_cast<const float*>(sRec + kLdsScales + R::kGamma - R::kScales);
     Split8 now, next, held;
     bf16x8 ka = operand(sK, 0), qa = operand(sQ, 0), q6;
     now.set(quad(st[0], 0), quad(st[0], 1));
@@ -559,7 +838,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     f32x16 vn;
     bf16x8 wt[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) wt[i] = weight(R::kT, 0, i);
+    for (int i = 0; i < 3; ++i) wt[i] = weight(kLdsT, 0, i);
     f32x4 sq[4], ck[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sq[q] = scales[R::kSq + 2 * q];
@@ -567,7 +846,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       if (i < 5) next.stage(i);
       if (i % 2 == 0) prefetch(3 + i / 2);
     };
-    LD_PRODUCTS(true, vn, held, slot_t0, R::kT, 1)
+    LD_PRODUCTS(true, vn, held, slot_t0, kLdsT, 1)
     auto slot_t1 = [&](int i) __attribute__((always_inline)) {
       if (i < 2) {
 #pragma unroll
@@ -579,7 +858,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
         normalise(i - 2);
       }
     };
-    LD_PRODUCTS(false, vn, next, slot_t1, R::kP, 0)
+    LD_PRODUCTS(false, vn, next, slot_t1, kLdsP, 0)
 #pragma unroll
     for (int q = 0; q < 2; ++q) ck[q] = scales[R::kCk + 2 * q];
     // beside P X: the split of ck V_new (now: step 0, last: step 1)
@@ -603,7 +882,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       }
       if (i >= 4) ck[i - 2] = scales[R::kCk + 2 * (i - 2)];
     };
-    LD_PRODUCTS(false, o, held, slot_p0, R::kP, 1)
+    LD_PRODUCTS(false, o, held, slot_p0, kLdsP, 1)
     auto slot_p1 = [&](int i) __attribute__((always_inline)) {
       if (i % 3 == 0) prefetch(8 + i / 3);
       if (i == 0)
@@ -611,7 +890,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       else
         last.stage(i - 1);
     };
-    LD_PRODUCTS(false, o, next, slot_p1, R::kP, 1)
+    LD_PRODUCTS(false, o, next, slot_p1, kLdsP, 1)
 #undef LD_PRODUCTS
     // S' = exp(G_n-1) S + K^T (ck V_new); beside it the raw outputs to LDS, rounded to bf16, and
     // the previous chunk's norm
@@ -668,20 +947,29 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
 
 }  // namespace
 
-int launch_chunk_heads(const DecodeParams& p, int num_sequences, const float* ws,
-                       const int32_t* chunk_start, int records, bool w_bf16, hipStream_t stream) {
+int launch_chunk_heads(const DecodeParams& p, int num_sequences, float* ws,
+                       const int32_t* chunk_start, int records, bool dt_bf16, bool w_bf16,
+                       hipStream_t stream) {
   const int64_t units = static_cast<int64_t>(num_sequences) * p.num_k_heads;
   const int64_t groups = (units + 7) / 8 * 8 * p.group;
-  if (groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
+  const int64_t prep_groups =
+      (static_cast<int64_t>(records) * p.num_k_heads + kPrepWaves - 1) / kPrepWaves;
+  if (groups > 0x7fffffff || prep_groups > 0x7fffffff)
+    return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
   const auto at16 = [](const void* base, int64_t row) {
     return (reinterpret_cast<uintptr_t>(base) & 15) == 0 && (row & 7) == 0;
   };
-  const bool wide = at16(p.qkv, p.qkv_row) && at16(p.gate, p.gate_row) && at16(p.out, 0);
+  const bool wide_qkv = at16(p.qkv, p.qkv_row);
+  const auto prep = dt_bf16 ? (wide_qkv ? chunk_prep_heads_kernel<true, true> : chunk_prep_heads_kernel<true, false>)
+                            : (wide_qkv ? chunk_prep_heads_kernel<false, true> : chunk_prep_heads_kernel<false, false>);
+  hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(64 * kPrepWaves), 0,
+                     stream, p, num_sequences, ws, chunk_start, records);
+  const bool wide = wide_qkv && at16(p.gate, p.gate_row) && at16(p.out, 0);
   const auto kernel = w_bf16 ? (wide ? chunk_heads_kernel<true, true> : chunk_heads_kernel<true, false>)
                              : (wide ? chunk_heads_kernel<false, true> : chunk_heads_kernel<false, false>);
   hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(kThreads), 0, stream, p,
                      num_sequences, ws, chunk_start, records);
-  return LD_OK;
+  return check_launch("ld_gdn_prefill (chunked)");
 }
 
 }  // namespace ld
