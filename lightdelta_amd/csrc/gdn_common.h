@@ -138,26 +138,6 @@ inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
   return 32;
 }
 
-// Workspace record of one (32-token chunk, v-head) for chunk_heads_kernel, offsets in bytes:
-// T = (I + A)^-1 diag(beta) and P = P0 T (32 x 32 fp32, lower triangular) as their exact bf16
-// planes in operand order.  Of a step u, a lane (hi, lj) of the product holds row lj, tokens
-// 16 u + 8 (e / 4) + 4 hi + e % 4, e < 8, as 16 bytes; plane i of step 0 is at 1024 i +
-// (32 hi + lj) * 16, of step 1 (whose rows below 16 are zeros and not stored) at 3072 + 512 i +
-// (16 hi + lj - 16) * 16.  Then the per-token scales in fp32 (offsets of kSq, .. in 16-byte
-// pieces from kScales) sq = rq scale exp(G), ck = rk exp(G_n-1 - G), ws = rk exp(G), and
-// exp(G_n-1).
-struct HeadRecord {
-  static constexpr int kTokens = 32;
-  static constexpr int kT = 0;
-  static constexpr int kP = 4608;
-  static constexpr int kScales = 9216;
-  static constexpr int kSq = 0;
-  static constexpr int kCk = 8;
-  static constexpr int kWs = 16;
-  static constexpr int kGamma = kScales + 384;
-  static constexpr int kBytes = 9728;
-};
-
 int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequences,
                                         int64_t num_v_heads);
 // chunk_tokens: 64 or 32
@@ -165,7 +145,10 @@ int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequence
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
                            bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
                            hipStream_t stream, bool* normed);
-int launch_chunk_heads(const DecodeParams& p, int num_sequences, float* ws,
+// The whole-head scan of 32-token chunks (prefill_heads.hip).  own: it prepares its chunks itself;
+// else a launch of its own does, into `records` records of kHeadRecordBytes at ws.
+constexpr int64_t kHeadRecordBytes = 9728;
+int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float* ws,
                        const int32_t* chunk_start, int records, bool dt_bf16, bool w_bf16,
                        hipStream_t stream);
 

@@ -1752,7 +1752,7 @@ int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
 // Workspace: the records, then chunk_start (num_sequences + 1 int32, rounded up to 256 B).
 // Sized for 64-token chunks, which covers 32-token ones: with S >= 1 sequences,
 // (T / 32 + S) R32 <= (2 (T / 64) + 1 + S) R32 <= (T / 64 + S) R64 as 2 R32 <= R64.
-static_assert(2 * Rec32::kSize <= kRecord && HeadRecord::kBytes <= Rec32::kSize * 4,
+static_assert(2 * Rec32::kSize <= kRecord && kHeadRecordBytes <= Rec32::kSize * 4,
               "32-token records fit the workspace");
 int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
@@ -1760,19 +1760,30 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
 
 // Which scan the 32-token form runs: chunk_heads_kernel (a whole head per workgroup, norm
 // fused) or chunk_scan32_kernel (a head's rows over four workgroups).  A chunk takes a lone
-// workgroup of the first 3.5 us and of the second 2.3 us, so with few (sequence, head) pairs
+// workgroup of the first 3.2 us and of the second 2.3 us, so with few (sequence, head) pairs
 // the second's chain is the shorter; from two chunks per CU on the first's throughput decides,
-// and for prompts of one or two chunks the launch it saves (us, first / second, at 32 v-heads:
-// 1 x 64 27 / 28, 1 x 256 46 / 35, 4 x 256 50.9 / 49.8, 4 x 1024 144 / 137, 5 x 1024 150 / 181,
-// 8 x 128 41 / 50, 8 x 1024 164 / 258, 32 x 1024 586 / 985, 1024 x 32 1264 / 1710).
+// and for short prompts the launches it saves (us, first / second, at 32 v-heads: 1 x 128 25 /
+// 27, 1 x 192 35 / 31, 2 x 128 25 / 29, 2 x 256 43 / 39, 4 x 192 37 / 42, 4 x 256 46 / 48,
+// 4 x 320 56 / 54, 4 x 1024 144 / 137, 5 x 1024 137 / 181, 8 x 1024 162 / 258, 32 x 1024 586 /
+// 985).
 bool whole_heads(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
-  return num_sequences * num_v_heads > 128 || num_tokens <= 64 * num_sequences;
+  const int64_t pairs = num_sequences * num_v_heads;
+  return pairs > 128 || num_tokens <= (pairs > 64 ? 256 : 128) * num_sequences;
 }
 
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
                   bool w_bf16, float* ws, int32_t* chunk_start, hipStream_t stream,
                   bool* normed) {
+  *normed = TT == 2 && whole_heads(num_tokens, num_sequences, p.num_v_heads);
+  // Short prompts' workgroups prepare their few chunks themselves: two launches fewer and no
+  // records in memory (us, with records / own: 1 x 64 26.5 / 19.7, 16 x 64 41.9 / 31.9, 8 x 128
+  // 39.5 / 28.4, 8 x 256 53.2 / 49.4, 32 x 256 169 / 155, 1024 x 32 1266 / 1196); over many
+  // chunks it lengthens the chain by 1 us a chunk (13 prompts up to 3000 tokens 265 / 338,
+  // 8 x 1024 161 / 177).
+  const bool own = num_tokens <= 256 * static_cast<int64_t>(num_sequences);
+  if (*normed && own)
+    return launch_chunk_heads(p, num_sequences, true, nullptr, nullptr, 0, dt_bf16, w_bf16, stream);
   constexpr int kCt = TT == 2 ? Rec32::kC : kC;
   const int64_t chunks = max_chunks<kCt>(num_tokens, num_sequences);
   if (chunks > 0x7fffffff || p.num_v_heads > 65535)
@@ -1783,8 +1794,9 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   const dim3 per_chunk(static_cast<uint32_t>(prep_groups));
   hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
                      num_sequences, chunk_start);
-  const bool heads = TT == 2 && whole_heads(num_tokens, num_sequences, p.num_v_heads);
-  *normed = heads;
+  if (*normed)
+    return launch_chunk_heads(p, num_sequences, false, ws, chunk_start, static_cast<int>(chunks),
+                              dt_bf16, w_bf16, stream);
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;
 #define LD_PREP_LAUNCH(K, D, W, N)                                                             \
@@ -1802,10 +1814,7 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
     else                                                                                       \
       LD_PREP_LAUNCH(K, false, false, N);                                                      \
   }
-  if (heads)
-    return launch_chunk_heads(p, num_sequences, ws, chunk_start, static_cast<int>(chunks), dt_bf16,
-                              w_bf16, stream);
-  if constexpr (TT == 2) {
+   if constexpr (TT == 2) {
     LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads)
   } else {
     LD_PREP_LAUNCHES(chunk_prep_kernel, kPrepThreads)

@@ -22,7 +22,8 @@
 //   S' = exp(G_n-1) S + K^T (ck V_new)   (24 products)
 // and the chunk's raw outputs go through LDS (bf16, the reference's rounding point) to the
 // gated RMSNorm of whole rows.  q, k and v come from qkv through LDS, the transposed operands
-// by ds_read_b64_tr_b16; T, P (as planes) and the per-token scales from the prep's records.
+// by ds_read_b64_tr_b16; T, P (as planes) and the per-token scales are prepared by the
+// workgroup itself (short prompts) or come as records from a launch ahead.
 //
 // What bounds it: vector issue and power.  A wave's chunk is 96 matrix instructions (3,072
 // cycles) and, with the norm, 880 vector ones (3,900 cycles of issue with the matrix ones');
@@ -44,13 +45,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTok = HeadRecord::kTokens;
+constexpr int kTok = 32;                       // tokens per chunk
 constexpr int kTileRow = kDim * 2;             // bytes of a q, k, v or raw-output row in LDS
 constexpr int kTileSize = kTok * kTileRow;
-// A chunk's record in LDS: T's and P's planes, plane i of step u at 3072 u + 1024 i, the scales.
-constexpr int kLdsT = 0;
-constexpr int kLdsP = 6144;
-constexpr int kLdsScales = 12288;
 
 // 16-byte pieces of row r are stored at piece ^ swizzle(r): a column of pieces over 16 rows
 // (operand A of the products with S) and 4 x 4 element blocks of 4 rows (transposed reads)
@@ -255,18 +252,43 @@ struct Norm {
   }
 };
 
-// ---- the records: one wave per (chunk, k-head) ------------------------------------------
-// A wave does a whole unit alone, so nothing waits on another wave: q and k come as operands of
-// v_mfma_f32_16x16x32_bf16 (for lane l, li = l % 16 and lg = l / 16: row 16 a + li, 16 bytes at
-// k = 32 s + 8 lg), which give the raw products K K^T and K Q^T below the diagonal and, from
-// the diagonals of K K^T and Q Q^T, the squared norms; then each v-head of the group in turn:
-// gates, -A to LDS, the inverses of I + A's two diagonal blocks (a column per lane), T10 =
-// -T1 A10 T0 and P = P0 T as 16 x 16 x 4 fp32 products with summation index k = 4 lg + step,
-// for which P0's tiles, T10 and the first product are operands as they are.
-// Bound by memory and by the latency of its chain: at 32 x 1024 tokens, 32 v-heads, 113 us for
-// 0.59 GB, where a workgroup of four waves with a barrier per phase took 169 us (0.69 GB, with
-// the planes' zero rows); at 512 prompts of 8 to 56 tokens 80 us against 132.
-constexpr int kPrepWaves = 4;
+// ---- a chunk's T, P and scales, by one wave ------------------------------------------------
+// Every fourth chunk each wave does one of the next four alone, so nothing waits on another
+// wave: q and k come as operands of v_mfma_f32_16x16x32_bf16 (for lane l, li = l % 16 and
+// lg = l / 16: row 16 a + li, 16 bytes at k = 32 s + 8 lg), which give the raw products K K^T
+// and K Q^T below the diagonal and, from the diagonals of K K^T and Q Q^T, the squared norms;
+// then the gates, -A to LDS, the inverses of I + A's two diagonal blocks (a column per lane),
+// T10 = -T1 A10 T0 and P = P0 T as 16 x 16 x 4 fp32 products with summation index k = 4 lg +
+// step, for which P0's tiles, T10 and the first product are operands as they are.
+
+// What the chunks' products read of it, in LDS, offsets in bytes: T = (I + A)^-1 diag(beta) and
+// P = P0 T (32 x 32 fp32, lower triangular) as their exact bf16 planes in operand order.  Of a
+// step u, a lane (hi, lj) of the product holds row lj, tokens 16 u + 8 (e / 4) + 4 hi + e % 4,
+// e < 8, as 16 bytes; plane i of step 0 is at 1024 i + (32 hi + lj) * 16, of step 1 (whose rows
+// below 16 are zeros and not stored) at 3072 + 512 i + (16 hi + lj - 16) * 16.  Then the
+// per-token scales in fp32 (offsets of kSq, .. in 16-byte pieces from kScales) sq = rq scale
+// exp(G), ck = rk exp(G_n-1 - G), ws = rk exp(G), and exp(G_n-1).
+struct Record {
+  static constexpr int kT = 0;
+  static constexpr int kP = 4608;
+  static constexpr int kScales = 9216;
+  static constexpr int kSq = 0;
+  static constexpr int kCk = 8;
+  static constexpr int kWs = 16;
+  static constexpr int kGamma = kScales + 384;
+  static constexpr int kBytes = static_cast<int>(kHeadRecordBytes);
+};
+
+// The wave's working memory, in the place of the planes it writes at the end.
+struct PrepScratch {
+  static constexpr int kARow = kTok + 4;   // padded rows (floats)
+  static constexpr int kTRow = 20;
+  float a[kTok][kARow];                    // -A
+  float t[3][16][kTRow];                   // T0, T1, T10
+  float g[kTok], glo[kTok];                // G / ln 2 as a sum of two floats
+  float beta[kTok], rq[kTok], rk[kTok];
+};
+static_assert(sizeof(PrepScratch) <= Record::kScales, "the scratch fits the planes' place");
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -280,90 +302,98 @@ __device__ __forceinline__ f32x4 mfma_f32(f32x4 a, f32x4 b, f32x4 c) {
   return c;
 }
 
-// Inclusive sums over the 32 lanes of each half wave (lane 32 + i as lane i).
-__device__ __forceinline__ float prefix_sum32(float x, int lane) {
-  x += dpp<0x111>(x);   // row_shr:1, 2, 4, 8: zeros from below the row
-  x += dpp<0x112>(x);
-  x += dpp<0x114>(x);
-  x += dpp<0x118>(x);
-  const float row0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 15));
-  return x + ((lane & 16) != 0 ? row0 : 0.0f);
+// Inclusive sums over the 32 lanes of each half wave (lane 32 + i as lane i), in 64 bits: decays
+// between two tokens are differences of these sums, and rounded to 32 bits the sums' error (half
+// an ulp of up to about 70) was most of the states': against 64 bits 1.9e-7 to 7.3e-7 over six
+// workloads, 0.9e-7 to 1.0e-7 this way.
+template <int Ctrl>
+__device__ __forceinline__ double dpp64(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), Ctrl, 0xF, 0xF, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), Ctrl, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+__device__ __forceinline__ double prefix_sum32(double x, int lane) {
+  x += dpp64<0x111>(x);   // row_shr:1, 2, 4, 8: zeros from below the row
+  x += dpp64<0x112>(x);
+  x += dpp64<0x114>(x);
+  x += dpp64<0x118>(x);
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(u), 15);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), 15);
+  const double row0 = __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+  return x + ((lane & 16) != 0 ? row0 : 0.0);
 }
 
-template <bool DtBf16, bool Wide>
-__global__ __launch_bounds__(64 * kPrepWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
-                             const int32_t* chunk_start, int records) {
-  using R = HeadRecord;
-  constexpr int kARow = kTok + 4;   // padded rows (floats)
-  constexpr int kTRow = 20;
-  struct Scratch {
-    float a[kTok][kARow];           // -A
-    float t[3][16][kTRow];          // T0, T1, T10
-    float g[kTok], beta[kTok], rq[kTok], rk[kTok];
-  };
-  __shared__ __attribute__((aligned(16))) Scratch scratch[kPrepWaves];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  Scratch& sc = scratch[wave];
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * kPrepWaves + wave;   // chunk * H + k-head
-  const int g = static_cast<int>(unit / p.num_k_heads);
-  if (g >= records) return;
-  const int key_head = static_cast<int>(unit - static_cast<int64_t>(g) * p.num_k_heads);
-  int seq = 0, t0 = 0, len = 0;
-  if (!find_chunk<kTok>(p.cu, chunk_start, num_sequences, g, seq, t0, len)) return;
+// q and k of one chunk as loaded (zeros past its end), and the gates of one v-head, of token
+// lane % 32.
+struct PrepInputs {
+  u32x4 q[2][4], k[2][4];
+};
+struct PrepGates {
+  uint16_t a, b;
+  float a_log, dt_bias;
+};
+
+template <bool Wide>
+__device__ __forceinline__ void prep_fetch(PrepInputs& x, const DecodeParams& p, int t0, int len,
+                                           int key_head, int lane) {
   const int li = lane & 15;
   const int lg = lane >> 4;
-
-  // a v-head's gate inputs, lane = token (lanes 32 .. 63 as 0 .. 31), fetched one v-head ahead
-  const int token = lane & 31;
-  uint16_t gate_a = 0, gate_b = 0;
-  float gate_a_log = 0.0f, gate_dt_bias = 0.0f;
-  auto fetch_gates = [&](int head) __attribute__((always_inline)) {
-    const int64_t tok = t0 + min(token, len - 1);
-    gate_a = p.a[tok * p.a_row + head];
-    gate_b = p.b[tok * p.b_row + head];
-    gate_a_log = p.a_log[head];
-    gate_dt_bias = load_param(p.dt_bias, head, DtBf16);
-  };
-  fetch_gates(key_head * p.group);
-
-  // raw tiles of the inputs (exact products, fp32 sums): kk[0, 1, 2] = K K^T (0,0), (1,0), (1,1),
-  // rows 4 lg + r, column li; kq = K Q^T of P's tiles (0,0), (1,0), (1,1): row li of P0, columns
-  // 4 lg + r
-  f32x4 kk[3], kq[3];
-  {
-    const uint32_t row_bytes = static_cast<uint32_t>(p.qkv_row) * 2;
-    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(p.qkv + static_cast<int64_t>(t0) * p.qkv_row), 0,
-        (len - 1) * static_cast<int>(row_bytes) + (2 * p.num_k_heads + p.num_v_heads) * kTileRow,
-        0x00020000);
-    u32x4 q[2][4], k[2][4];   // zeros past the chunk's end
+  const uint32_t row_bytes = static_cast<uint32_t>(p.qkv_row) * 2;
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(p.qkv + static_cast<int64_t>(t0) * p.qkv_row), 0,
+      (len - 1) * static_cast<int>(row_bytes) + (2 * p.num_k_heads + p.num_v_heads) * kTileRow,
+      0x00020000);
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const uint32_t at = 16 * a + li < len ? (16 * a + li) * row_bytes + lg * 16 : 0xfffff000u;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        k[a][s] = load_piece<Wide>(rows, at, (p.num_k_heads + key_head) * kTileRow + s * 64);
-        q[a][s] = load_piece<Wide>(rows, at, key_head * kTileRow + s * 64);
-      }
-    }
-    f32x4 qq[2];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) kk[i] = kq[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    qq[0] = qq[1] = kk[0];
+  for (int a = 0; a < 2; ++a) {
+    const uint32_t at = 16 * a + li < len ? (16 * a + li) * row_bytes + lg * 16 : 0xfffff000u;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const bf16x8 k0 = __builtin_bit_cast(bf16x8, k[0][s]);
-      const bf16x8 k1 = __builtin_bit_cast(bf16x8, k[1][s]);
-      const bf16x8 q0 = __builtin_bit_cast(bf16x8, q[0][s]);
-      const bf16x8 q1 = __builtin_bit_cast(bf16x8, q[1][s]);
-      kk[0] = mfma16(k0, k0, kk[0]);
-      kk[1] = mfma16(k1, k0, kk[1]);
-      kk[2] = mfma16(k1, k1, kk[2]);
-      kq[0] = mfma16(k0, q0, kq[0]);
-      kq[1] = mfma16(k0, q1, kq[1]);
-      kq[2] = mfma16(k1, q1, kq[2]);
+      x.k[a][s] = load_piece<Wide>(rows, at, (p.num_k_heads + key_head) * kTileRow + s * 64);
+      x.q[a][s] = load_piece<Wide>(rows, at, key_head * kTileRow + s * 64);
+    }
+  }
+}
+
+template <bool DtBf16>
+__device__ __forceinline__ void prep_gates(PrepGates& x, const DecodeParams& p, int t0, int len,
+                                           int head, int lane) {
+  const int64_t tok = t0 + min(lane & 31, len - 1);
+  x.a = p.a[tok * p.a_row + head];
+  x.b = p.b[tok * p.b_row + head];
+  x.a_log = p.a_log[head];
+  x.dt_bias = load_param(p.dt_bias, head, DtBf16);
+}
+
+// kk: raw tiles of K K^T (0,0), (1,0), (1,1), rows 4 lg + r, column li; kq: K Q^T of P's tiles
+// (0,0), (1,0), (1,1): row li of P0, columns 4 lg + r (exact products, fp32 sums).
+struct PrepTiles {
+  f32x4 kk[3], kq[3];
+};
+
+// The part that depends on q and k alone: the raw tiles, and the inverse norms to the scratch.
+__device__ __forceinline__ void prep_tiles(PrepTiles& x, const PrepInputs& in, float scale, int len,
+                                           PrepScratch& sc, int lane) {
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  {
+    f32x4 qq[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) x.kk[i] = x.kq[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    qq[0] = qq[1] = x.kk[0];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bf16x8 k0 = __builtin_bit_cast(bf16x8, in.k[0][s]);
+      const bf16x8 k1 = __builtin_bit_cast(bf16x8, in.k[1][s]);
+      const bf16x8 q0 = __builtin_bit_cast(bf16x8, in.q[0][s]);
+      const bf16x8 q1 = __builtin_bit_cast(bf16x8, in.q[1][s]);
+      x.kk[0] = mfma16(k0, k0, x.kk[0]);
+      x.kk[1] = mfma16(k1, k0, x.kk[1]);
+      x.kk[2] = mfma16(k1, k1, x.kk[2]);
+      x.kq[0] = mfma16(k0, q0, x.kq[0]);
+      x.kq[1] = mfma16(k0, q1, x.kq[1]);
+      x.kq[2] = mfma16(k1, q1, x.kq[2]);
       qq[0] = mfma16(q0, q0, qq[0]);
       qq[1] = mfma16(q1, q1, qq[1]);
     }
@@ -373,45 +403,52 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
         const f32x4 dq = qq[a];
-        const f32x4 dk = kk[2 * a];
+        const f32x4 dk = x.kk[2 * a];
         const int r = li & 3;
         const float q2 = r < 2 ? (r == 0 ? dq[0] : dq[1]) : (r == 2 ? dq[2] : dq[3]);
         const float k2 = r < 2 ? (r == 0 ? dk[0] : dk[1]) : (r == 2 ? dk[2] : dk[3]);
         const bool live = 16 * a + li < len;
-        sc.rq[16 * a + li] = live ? fast_rsqrt(q2 + 1e-6f) * p.scale : 0.0f;
+        sc.rq[16 * a + li] = live ? fast_rsqrt(q2 + 1e-6f) * scale : 0.0f;
         sc.rk[16 * a + li] = live ? fast_rsqrt(k2 + 1e-6f) : 0.0f;
       }
     }
   }
-  lds_order();
+}
 
+// One v-head's T, P and scales to `rec` (in LDS, where the scratch may be in the planes' place,
+// or in memory).
+__device__ __forceinline__ void prep_head(const PrepTiles& x, const PrepGates& in, int len,
+                                          PrepScratch& sc, uint8_t* rec, int lane) {
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int token = lane & 31;
   const auto at4 = [](const float* x) __attribute__((always_inline)) {
     return *reinterpret_cast<const f32x4*>(x);
   };
-  for (int member = 0; member < p.group; ++member) {
-    const int head = key_head * p.group + member;
-    uint8_t* const rec = reinterpret_cast<uint8_t*>(ws) +
-                         (static_cast<int64_t>(g) * p.num_v_heads + head) * R::kBytes;
+  {
     // gates and the in-chunk cumulative log decay: the token-serial form's arithmetic
     {
       const bool live = token < len;
-      const float x = bf16_to_f32(gate_a) + gate_dt_bias;
-      const float gl = live ? -__expf(gate_a_log) * softplus(x) : 0.0f;
-      const float beta = live ? sigmoid(bf16_to_f32(gate_b)) : 0.0f;
-      if (member + 1 < p.group) fetch_gates(head + 1);
-      const float G = prefix_sum32(gl, lane);
-      const float glast = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(G), 31));
-      const float eg = __expf(G);
+      const float xa = bf16_to_f32(in.a) + in.dt_bias;
+      const float gl = live ? -__expf(in.a_log) * softplus(xa) : 0.0f;
+      const float beta = live ? sigmoid(bf16_to_f32(in.b)) : 0.0f;
+      const double sum = prefix_sum32(gl, lane) * 1.4426950408889634;   // exp2 from here on
+      const float G = static_cast<float>(sum);
+      const float glo = static_cast<float>(sum - static_cast<double>(G));
+      const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(G), 31));
+      const float last_lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(glo), 31));
+      const float eg = __builtin_amdgcn_exp2f(G);
       const float rk = sc.rk[token];
-      float* const scales = reinterpret_cast<float*>(rec + R::kScales);
+      float* const scales = reinterpret_cast<float*>(rec + Record::kScales);
       if (lane < kTok) {
         sc.g[token] = G;
+        sc.glo[token] = glo;
         sc.beta[token] = beta;
-        scales[4 * R::kSq + token] = sc.rq[token] * eg;
-        scales[4 * R::kWs + token] = eg * rk;
+        scales[4 * Record::kSq + token] = sc.rq[token] * eg;
+        scales[4 * Record::kWs + token] = eg * rk;
       } else {
-        scales[4 * R::kCk + token] = rk * __expf(glast - G);
-        if (token == 0) *reinterpret_cast<float*>(rec + R::kGamma) = __expf(glast);
+        scales[4 * Record::kCk + token] = rk * __builtin_amdgcn_exp2f((last - G) + (last_lo - glo));
+        if (token == 0) *reinterpret_cast<float*>(rec + Record::kGamma) = __builtin_amdgcn_exp2f(last);
       }
     }
     lds_order();
@@ -422,14 +459,16 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
       const int mt = i > 0 ? 1 : 0, nt = i > 1 ? 1 : 0;
       const int mcol = 16 * nt + li;
       const float gm = sc.g[mcol];
+      const float glm = sc.glo[mcol];
       const float rkm = sc.rk[mcol];
       const f32x4 gi = at4(&sc.g[16 * mt + 4 * lg]);
+      const f32x4 gli = at4(&sc.glo[16 * mt + 4 * lg]);
       const f32x4 bi = at4(&sc.beta[16 * mt + 4 * lg]);
       const f32x4 rki = at4(&sc.rk[16 * mt + 4 * lg]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = -(bi[r] * __expf(gi[r] - gm) * ((rki[r] * rkm) * kk[i][r]));
-        sc.a[16 * mt + 4 * lg + r][mcol] = i == 1 || li < 4 * lg + r ? x : 0.0f;
+        const float na = -(bi[r] * __builtin_amdgcn_exp2f((gi[r] - gm) + (gli[r] - glm)) * ((rki[r] * rkm) * x.kk[i][r]));
+        sc.a[16 * mt + 4 * lg + r][mcol] = i == 1 || li < 4 * lg + r ? na : 0.0f;
       }
     }
     // P0's tiles: row li, columns 4 lg + r
@@ -438,13 +477,15 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
     for (int i = 0; i < 3; ++i) {
       const int mt = i > 0 ? 1 : 0, nt = i > 1 ? 1 : 0;
       const float gi = sc.g[16 * mt + li];
+      const float gli = sc.glo[16 * mt + li];
       const float rqi = sc.rq[16 * mt + li];
       const f32x4 gm = at4(&sc.g[16 * nt + 4 * lg]);
+      const f32x4 glm = at4(&sc.glo[16 * nt + 4 * lg]);
       const f32x4 rkm = at4(&sc.rk[16 * nt + 4 * lg]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = __expf(gi - gm[r]) * ((rqi * rkm[r]) * kq[i][r]);
-        p0[i][r] = (i == 1 || 4 * lg + r <= li) && 16 * mt + li < len ? x : 0.0f;
+        const float pv = __builtin_amdgcn_exp2f((gi - gm[r]) + (gli - glm[r])) * ((rqi * rkm[r]) * x.kq[i][r]);
+        p0[i][r] = (i == 1 || 4 * lg + r <= li) && 16 * mt + li < len ? pv : 0.0f;
       }
     }
     lds_order();
@@ -459,7 +500,7 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
 #pragma unroll
       for (int mc = 0; mc < 15; ++mc)
 #pragma unroll
-        for (int i = mc + 1; i < 16; ++i) col[i] = fmaf(ab[i * kARow + mc], col[mc], col[i]);
+        for (int i = mc + 1; i < 16; ++i) col[i] = fmaf(ab[i * PrepScratch::kARow + mc], col[mc], col[i]);
       if (lane < 32) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc.t[block][i][li] = col[i];
@@ -489,6 +530,7 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
     const f32x4 t10r = at4(&sc.t[2][li][4 * lg]);
     const f32x4 b0 = at4(&sc.beta[4 * lg]);
     const f32x4 b1 = at4(&sc.beta[16 + 4 * lg]);
+    lds_order();   // the planes may take the scratch's place: its last reads are above
     // to the planes: tile (mt, nt), row li, columns 4 lg ..
     auto put = [&](int base, int mt, int nt, f32x4 x) __attribute__((always_inline)) {
       const Split4 sp = split4(x);
@@ -498,22 +540,62 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
       for (int pl = 0; pl < 3; ++pl)
         *reinterpret_cast<uint2*>(at + pl * (nt == 0 ? 1024 : 512)) = sp.p[pl];
     };
-    put(R::kT, 0, 0, t0r * b0);
-    put(R::kT, 1, 0, t10r * b0);
-    put(R::kT, 1, 1, t1r * b1);
-    put(R::kP, 0, 0, pt[0] * b0);
-    put(R::kP, 1, 0, pt[1] * b0);
-    put(R::kP, 1, 1, pt[2] * b1);
+    put(Record::kT, 0, 0, t0r * b0);
+    put(Record::kT, 1, 0, t10r * b0);
+    put(Record::kT, 1, 1, t1r * b1);
+    put(Record::kP, 0, 0, pt[0] * b0);
+    put(Record::kP, 1, 0, pt[1] * b0);
+    put(Record::kP, 1, 1, pt[2] * b1);
+  }
+}
+
+// The records of every chunk in a launch of their own, one wave per (chunk, k-head) running the
+// group's v-heads in turn: for longer prompts, where a head's workgroup would do its chunks'
+// preparation in its own chain.  Bound by memory and by the latency of a unit's chain: at
+// 32 x 1024 tokens, 32 v-heads, 114 us for 0.59 GB (134 us at four waves a SIMD, which spills),
+// where a workgroup of four waves with a barrier per phase took 169 us (0.69 GB, with the
+// planes' zero rows and the decay's sums in 32 bits).
+template <bool DtBf16, bool Wide>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
+void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
+                             const int32_t* chunk_start, int records) {
+  __shared__ __attribute__((aligned(16))) PrepScratch scratch[kWaves];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int64_t unit = static_cast<int64_t>(blockIdx.x) * kWaves + wave;   // chunk * H + k-head
+  const int g = static_cast<int>(unit / p.num_k_heads);
+  if (g >= records) return;
+  const int key_head = static_cast<int>(unit - static_cast<int64_t>(g) * p.num_k_heads);
+  int seq = 0, t0 = 0, len = 0;
+  if (!find_chunk<kTok>(p.cu, chunk_start, num_sequences, g, seq, t0, len)) return;
+  PrepScratch& sc = scratch[wave];
+  PrepGates gates, next;
+  prep_gates<DtBf16>(next, p, t0, len, key_head * p.group, lane);
+  PrepTiles tiles;
+  {
+    PrepInputs in;
+    prep_fetch<Wide>(in, p, t0, len, key_head, lane);
+    prep_tiles(tiles, in, p.scale, len, sc, lane);
+  }
+  for (int member = 0; member < p.group; ++member) {
+    const int head = key_head * p.group + member;
+    gates = next;
+    if (member + 1 < p.group) prep_gates<DtBf16>(next, p, t0, len, head + 1, lane);
+    lds_order();
+    prep_head(tiles, gates, len, sc,
+              reinterpret_cast<uint8_t*>(ws) +
+                  (static_cast<int64_t>(g) * p.num_v_heads + head) * Record::kBytes, lane);
     lds_order();   // (the next v-head rewrites the scratch)
   }
 }
 
-// Wide: the rows of qkv, gate and out start at 16-byte boundaries.
-template <bool WBf16, bool Wide>
+// Own: the workgroup prepares its chunks itself (no workspace), a wave per chunk, four at a
+// time; else their records are in `ws`.
+template <bool Own, bool DtBf16, bool WBf16, bool Wide>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws,
                         const int32_t* chunk_start, int records) {
-  using R = HeadRecord;
+  using R = Record;
   // Workgroups go to the 8 XCDs round-robin by id; the v-heads of one (sequence, k-head) read
   // the same q and k, so they are given ids on one XCD.
   const int xcd = blockIdx.x & 7;
@@ -532,16 +614,23 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   const int eos = p.cu[seq + 1];
   const int slot = p.indices[seq];
   const bool from_slot = slot > 0 && p.has_initial[seq] != 0;
-  const int gbase = chunk_start[seq];
+  const int gbase = Own ? 0 : chunk_start[seq];
   // (bounded by the records the workspace holds, whatever cu_seqlens says)
-  const int chunks = min((eos - bos + kTok - 1) / kTok, max(records - gbase, 0));
+  const int chunks = min((eos - bos + kTok - 1) / kTok, Own ? 0x7fffffff : max(records - gbase, 0));
 
+  constexpr int kRing = Own ? kWaves : 1;
+  // In LDS a record is as it was prepared (Own), its step 1 zeroed as it is read, or, where the
+  // room is there, with the zero rows: T's and P's plane i of step u at 3072 u + 1024 i (7 us of
+  // 583 at 32 x 1024).
+  constexpr int kLdsP = Own ? R::kP : 6144;
+  constexpr int kLdsScales = Own ? R::kScales : 12288;
+  constexpr int kLdsRecord = kLdsScales + R::kBytes - R::kScales;
   __shared__ __attribute__((aligned(16))) uint8_t sK[kTileSize];
   __shared__ __attribute__((aligned(16))) uint8_t sQ[kTileSize];
   // v of the chunk, then in its place the raw outputs (a wave reads and writes its own 32
   // columns of both); two, as the norm reads one while the next chunk's v arrives
   __shared__ __attribute__((aligned(16))) uint8_t sV[2][kTileSize];
-  __shared__ __attribute__((aligned(16))) uint8_t sRec[kLdsScales + R::kBytes - R::kScales];
+  __shared__ __attribute__((aligned(16))) uint8_t sRec[kRing][kLdsRecord];   // chunk c's in c % kRing
   __shared__ __attribute__((aligned(16))) float sW[kDim];
 
   if (tid < kDim) sW[tid] = load_param(p.norm_weight, tid, WBf16);
@@ -556,9 +645,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   const int v_col = (2 * p.num_k_heads + head) * kTileRow;
   const int qkv_bytes = (2 * p.num_k_heads + p.num_v_heads) * kTileRow;
   const uint32_t dst = srow * kTileRow + ((spiece ^ swizzle(srow)) << 4);
-  // where the record's bytes go in LDS: both steps' planes whole there (1024 bytes each), step
-  // 1's upper rows zeroed once
-  auto lds_at = [](int byte) __attribute__((always_inline)) {
+  auto lds_at = [](int byte) __attribute__((always_inline)) {   // of a record's byte (not Own)
     const int base = byte < R::kP ? 0 : kLdsP;
     const int at = byte < R::kP ? byte : byte - R::kP;
     const int step1 = at - 3072;
@@ -567,15 +654,17 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   };
   const int rec_at[2] = {lds_at(tid * 16), lds_at(4096 + tid * 16)};
   const int rest_at = lds_at(8192 + tid * 4);
-  for (int i = tid; i < 2 * 3 * 2 * 16; i += kThreads)   // matrix, plane, hi, 16-byte piece
-    *reinterpret_cast<u32x4*>(sRec + (i / 96) * kLdsP + 3072 + ((i / 32) % 3) * 1024 +
-                              ((i >> 4) & 1) * 512 + (i & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
+  if constexpr (!Own) {
+    for (int i = tid; i < 2 * 3 * 2 * 16; i += kThreads)   // matrix, plane, hi, 16-byte piece
+      *reinterpret_cast<u32x4*>(sRec[0] + (i / 96) * kLdsP + 3072 + ((i / 32) % 3) * 1024 +
+                                ((i >> 4) & 1) * 512 + (i & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
+  }
   struct Staged {
     u32x4 q[2], k[2], v[2], rec[2];
-    uint32_t rest, scales;   // the planes' last KiB and the scales, a word per thread
+    uint32_t rest[2];   // the record's last 1.5 KiB
   };
   // Where chunk c's operands are (past the last chunk: resources over 0 bytes, whose loads
-  // return zeros), and its load i of 10.
+  // return zeros), and its load i of 6 (Own) or 10.
   struct Source {
     __amdgpu_buffer_rsrc_t rows, rec;
     uint32_t at[2];
@@ -587,10 +676,11 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     x.rows = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.qkv + static_cast<int64_t>(t0) * p.qkv_row), 0,
         live > 0 ? (live - 1) * static_cast<int>(row_bytes) + qkv_bytes : 0, 0x00020000);
-    x.rec = record_resource(
-        ws + (static_cast<int64_t>(gbase + min(c, max(chunks - 1, 0))) * p.num_v_heads + head) *
-                 (R::kBytes / 4),
-        c < chunks ? R::kBytes : 0);
+    if constexpr (!Own)
+      x.rec = record_resource(
+          ws + (static_cast<int64_t>(gbase + min(c, max(chunks - 1, 0))) * p.num_v_heads + head) *
+                   (R::kBytes / 4),
+          c < chunks ? R::kBytes : 0);
     // rows past the chunk's end: an offset past the resource, so zeros
 #pragma unroll
     for (int i = 0; i < 2; ++i) x.at[i] = srow + 16 * i < live ? src + i * 16 * row_bytes : 0xfffff000u;
@@ -603,12 +693,12 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       x.q[i - 2] = load_piece<Wide>(from.rows, from.at[i - 2], q_col);
     else if (i < 6)
       x.v[i - 4] = load_piece<Wide>(from.rows, from.at[i - 4], v_col);
+    else if (Own)
+      return;
     else if (i < 8)
       x.rec[i - 6] = load16u(from.rec, tid * 16 + (i - 6) * 4096, 0);
-    else if (i == 8)
-      x.rest = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + 8192, 0, 0);
-    else
-      x.scales = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + R::kScales, 0, 0);
+    else   // (past the record's end: zeros)
+      x.rest[i - 8] = __builtin_amdgcn_raw_buffer_load_b32(from.rec, tid * 4 + 8192 + (i - 8) * 1024, 0, 0);
   };
   auto put = [&](const Staged& x, int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -617,21 +707,41 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       *reinterpret_cast<u32x4*>(sQ + dst + i * 16 * kTileRow) = x.q[i];
       *reinterpret_cast<u32x4*>(sV[buf] + dst + i * 16 * kTileRow) = x.v[i];
     }
+    if constexpr (!Own) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sRec + rec_at[i]) = x.rec[i];
-    *reinterpret_cast<uint32_t*>(sRec + rest_at) = x.rest;
-    if (tid < (R::kBytes - R::kScales) / 4)
-      *reinterpret_cast<uint32_t*>(sRec + kLdsScales + tid * 4) = x.scales;
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sRec[0] + rec_at[i]) = x.rec[i];
+      *reinterpret_cast<uint32_t*>(sRec[0] + rest_at) = x.rest[0];
+      if (tid < (R::kBytes - R::kScales) / 4)
+        *reinterpret_cast<uint32_t*>(sRec[0] + kLdsScales + tid * 4) = x.rest[1];
+    }
   };
-  static_assert(R::kScales == 2 * 4096 + 1024 && R::kBytes - R::kScales <= kThreads * 4,
-                "two pieces, a word and a scale per thread");
+  static_assert(R::kScales == 8192 + 1024 && R::kBytes - R::kScales <= 1024, "the record's loads");
 
+  // The chunk that this wave prepares first: its loads go out ahead of the state's and return
+  // first.
+  PrepInputs first;
+  PrepGates first_gates;
+  auto prep_rows = [&](int c) __attribute__((always_inline)) { return min(kTok, eos - bos - c * kTok); };
+  auto prepare_fetch = [&](PrepInputs& in, PrepGates& gates, int c) __attribute__((always_inline)) {
+    prep_fetch<Wide>(in, p, bos + c * kTok, prep_rows(c), key_head, lane);
+    prep_gates<DtBf16>(gates, p, bos + c * kTok, prep_rows(c), head, lane);
+  };
+  auto prepare = [&](const PrepInputs& in, const PrepGates& gates, int c) __attribute__((always_inline)) {
+    PrepScratch& sc = *reinterpret_cast<PrepScratch*>(sRec[w & (kRing - 1)]);
+    PrepTiles tiles;
+    prep_tiles(tiles, in, p.scale, prep_rows(c), sc, lane);
+    lds_order();
+    prep_head(tiles, gates, prep_rows(c), sc, sRec[w & (kRing - 1)], lane);
+  };
+  if (Own && w < chunks) prepare_fetch(first, first_gates, w);
+  asm volatile("" ::: "memory");
   Staged staged;
   if (chunks > 0) {
     const Source from = source(0);
 #pragma unroll
     for (int i = 0; i < 10; ++i) fetch(staged, from, i);
   }
+  asm volatile("" ::: "memory");
 
   // st[T][8 u + 4 h + r] = S[32 w + lj][32 T + 16 u + 8 hi + 4 h + r]
   f32x16 st[4];
@@ -662,8 +772,6 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
   // raw outputs: row 8 q + 4 hi + e, column 32 w + lj   ^ (e << 6) ^ ((q & 1) << 5)
   const uint32_t raw_at =
       4 * hi * kTileRow + (((4 * w + (lj >> 3)) ^ hi) << 4) + (lj & 7) * 2;
-  const uint8_t* const planes = sRec + lane * 16;
-  const f32x4* const scales = reinterpret_cast<const f32x4*>(sRec + kLdsScales) + hi;
 
   // The norm of chunk c - 1 runs beside chunk c's products; thread = (token, 16 columns).
   // Resources over the chunk's rows of gate and out (before the first chunk: over 0 bytes,
@@ -680,11 +788,11 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
         const_cast<uint16_t*>(base + static_cast<int64_t>(t0) * row + static_cast<int64_t>(head) * kDim),
         0, c >= 0 ? (min(kTok, eos - t0) - 1) * static_cast<int>(row * 2) + kTileRow : 0, 0x00020000);
   };
-  auto load_gate = [&](Norm& norm, int c) __attribute__((always_inline)) {
+  auto load_gate = [&](u32x4 (&to)[2], int c) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rows = chunk_rows(p.gate, p.gate_row, c);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      norm.gate[i] = load_piece<Wide>(rows, ntok * gate_bytes + ncol * 2 + 16 * i, 0);
+      to[i] = load_piece<Wide>(rows, ntok * gate_bytes + ncol * 2 + 16 * i, 0);
   };
   auto store_norm = [&](const Norm& norm, int c) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rows = chunk_rows(p.out, static_cast<int64_t>(p.num_v_heads) * kDim, c);
@@ -703,12 +811,23 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     }
   };
 
+  if (Own && w < chunks) prepare(first, first_gates, w);
   // (the state's loads are waited for here: inside the loop the waits would be counted
   // against later chunks' loads)
 #pragma unroll
   for (int T = 0; T < 4; ++T) pin(st[T]);
+  Norm norm;
+  u32x4 gate[2] = {};   // of the chunk whose raw outputs are next to be normalised
   for (int c = 0; c < chunks; ++c) {
     const int buf = c & 1;
+    if (Own && c > 0 && (c & (kWaves - 1)) == 0 && c + w < chunks) {
+      PrepInputs in;
+      PrepGates gates;
+      prepare_fetch(in, gates, c + w);
+      prepare(in, gates, c + w);
+    }
+    const uint8_t* const rec = sRec[c & (kRing - 1)];
+    const f32x4* const scales = reinterpret_cast<const f32x4*>(rec + kLdsScales) + hi;
     put(staged, buf);
     lds_barrier();   // the chunk's operands and the previous chunk's raw outputs are in LDS
 
@@ -720,8 +839,6 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       fetch(staged, from, i);
       asm volatile("" ::: "memory");
     };
-    Norm norm;
-    load_gate(norm, c - 1);
     const uint8_t* const last_raw = sV[buf ^ 1];
     auto normalise = [&](int i) __attribute__((always_inline)) {
       norm.slice(i, last_raw + raw0_at, last_raw + raw1_at, sW + ncol, p.eps);
@@ -735,7 +852,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     auto operand = [&](const uint8_t* tile, int n) __attribute__((always_inline)) {
       return *reinterpret_cast<const bf16x8*>(tile + (a_at ^ (n << 5)));
     };
-    const float gamma = *reinterpret_cast<const float*>(sRec + kLdsScales + R::kGamma - R::kScales);
+    const float gamma = *reinterpret_cast<const float*>(rec + kLdsScales + R::kGamma - R::kScales);
     Split8 now, next, held;
     bf16x8 ka = operand(sK, 0), qa = operand(sQ, 0), q6;
     now.set(quad(st[0], 0), quad(st[0], 1));
@@ -824,7 +941,12 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     // V_new = T X and O = diag(sq) O + P X, T and P as planes (held, next: X's), the smallest
     // products of a step first
     auto weight = [&](int base, int u, int i) __attribute__((always_inline)) {
-      return *reinterpret_cast<const bf16x8*>(planes + base + (3 * u + i) * 1024);
+      if (u == 0 || !Own)
+        return *reinterpret_cast<const bf16x8*>(rec + base + u * 3072 + i * 1024 + lane * 16);
+      u32x4 x = *reinterpret_cast<const u32x4*>(rec + base + 3072 + i * 512 + (16 * hi + (lj & 15)) * 16);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) x[d] = lj < 16 ? 0u : x[d];   // rows above the triangle
+      return __builtin_bit_cast(bf16x8, x);
     };
     // the six products of a step; NEXT, UN: the matrix and step whose planes replace the
     // current ones as they fall free
@@ -838,7 +960,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     f32x16 vn;
     bf16x8 wt[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) wt[i] = weight(kLdsT, 0, i);
+    for (int i = 0; i < 3; ++i) wt[i] = weight(R::kT, 0, i);
     f32x4 sq[4], ck[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sq[q] = scales[R::kSq + 2 * q];
@@ -846,7 +968,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       if (i < 5) next.stage(i);
       if (i % 2 == 0) prefetch(3 + i / 2);
     };
-    LD_PRODUCTS(true, vn, held, slot_t0, kLdsT, 1)
+    LD_PRODUCTS(true, vn, held, slot_t0, R::kT, 1)
     auto slot_t1 = [&](int i) __attribute__((always_inline)) {
       if (i < 2) {
 #pragma unroll
@@ -871,7 +993,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       to.set(lo, hi);
     };
     auto slot_p0 = [&](int i) __attribute__((always_inline)) {
-      if (i % 3 == 0) prefetch(6 + i / 3);
+      if (!Own && i % 3 == 0) prefetch(6 + i / 3);
       if (i == 0) {
         normalise(4);
       } else if (i == 1) {
@@ -884,7 +1006,7 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     };
     LD_PRODUCTS(false, o, held, slot_p0, kLdsP, 1)
     auto slot_p1 = [&](int i) __attribute__((always_inline)) {
-      if (i % 3 == 0) prefetch(8 + i / 3);
+      if (!Own && i % 3 == 0) prefetch(8 + i / 3);
       if (i == 0)
         scaled_vn(2, last);
       else
@@ -900,6 +1022,11 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       const bf16x4 k1 = read_tr(sK + (kt_at ^ (T << 6) ^ (1 << 5)) + (16 * u + 8) * kTileRow);
       return __builtin_shufflevector(k0, k1, 0, 1, 2, 3, 4, 5, 6, 7);
     };
+    norm.gate[0] = gate[0];
+    norm.gate[1] = gate[1];
+    asm volatile("" ::: "memory");
+    load_gate(gate, c);
+    asm volatile("" ::: "memory");
     bf16x8 kt = key_t(0);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -924,16 +1051,6 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
     store_norm(norm, c - 1);
     lds_barrier();   // every read of the operands is done
   }
-  if (chunks > 0) {   // the last chunk's norm (its raw outputs are complete past the barrier)
-    Norm norm;
-    load_gate(norm, chunks - 1);
-    const uint8_t* const last_raw = sV[(chunks - 1) & 1];
-#pragma unroll
-    for (int i = 0; i < 23; ++i)
-      norm.slice(i, last_raw + raw0_at, last_raw + raw1_at, sW + ncol, p.eps);
-    store_norm(norm, chunks - 1);
-  }
-
   if (slot > 0) {
     float* tile = p.state + static_cast<int64_t>(slot) * p.state_slot +
                   static_cast<int64_t>(head) * kDim * kDim + (32 * w + lj) * kDim + 8 * hi;
@@ -943,30 +1060,43 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4*>(tile + 32 * T + 16 * (q >> 1) + 4 * (q & 1)) = quad(st[T], q);
   }
+  if (chunks > 0) {   // the last chunk's norm (its raw outputs are complete past the barrier)
+    norm.gate[0] = gate[0];
+    norm.gate[1] = gate[1];
+    const uint8_t* const last_raw = sV[(chunks - 1) & 1];
+#pragma unroll
+    for (int i = 0; i < 23; ++i)
+      norm.slice(i, last_raw + raw0_at, last_raw + raw1_at, sW + ncol, p.eps);
+    store_norm(norm, chunks - 1);
+  }
 }
 
 }  // namespace
 
-int launch_chunk_heads(const DecodeParams& p, int num_sequences, float* ws,
+int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float* ws,
                        const int32_t* chunk_start, int records, bool dt_bf16, bool w_bf16,
                        hipStream_t stream) {
   const int64_t units = static_cast<int64_t>(num_sequences) * p.num_k_heads;
   const int64_t groups = (units + 7) / 8 * 8 * p.group;
-  const int64_t prep_groups =
-      (static_cast<int64_t>(records) * p.num_k_heads + kPrepWaves - 1) / kPrepWaves;
+  const int64_t prep_groups = (static_cast<int64_t>(records) * p.num_k_heads + kWaves - 1) / kWaves;
   if (groups > 0x7fffffff || prep_groups > 0x7fffffff)
     return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
   const auto at16 = [](const void* base, int64_t row) {
     return (reinterpret_cast<uintptr_t>(base) & 15) == 0 && (row & 7) == 0;
   };
   const bool wide_qkv = at16(p.qkv, p.qkv_row);
-  const auto prep = dt_bf16 ? (wide_qkv ? chunk_prep_heads_kernel<true, true> : chunk_prep_heads_kernel<true, false>)
-                            : (wide_qkv ? chunk_prep_heads_kernel<false, true> : chunk_prep_heads_kernel<false, false>);
-  hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(64 * kPrepWaves), 0,
-                     stream, p, num_sequences, ws, chunk_start, records);
   const bool wide = wide_qkv && at16(p.gate, p.gate_row) && at16(p.out, 0);
-  const auto kernel = w_bf16 ? (wide ? chunk_heads_kernel<true, true> : chunk_heads_kernel<true, false>)
-                             : (wide ? chunk_heads_kernel<false, true> : chunk_heads_kernel<false, false>);
+#define LD_HEADS(O, D, W) (wide ? chunk_heads_kernel<O, D, W, true> : chunk_heads_kernel<O, D, W, false>)
+  const auto kernel = !own      ? (w_bf16 ? LD_HEADS(false, false, true) : LD_HEADS(false, false, false))
+                      : dt_bf16 ? (w_bf16 ? LD_HEADS(true, true, true) : LD_HEADS(true, true, false))
+                                : (w_bf16 ? LD_HEADS(true, false, true) : LD_HEADS(true, false, false));
+#undef LD_HEADS
+  if (!own) {
+    const auto prep = dt_bf16 ? (wide_qkv ? chunk_prep_heads_kernel<true, true> : chunk_prep_heads_kernel<true, false>)
+                              : (wide_qkv ? chunk_prep_heads_kernel<false, true> : chunk_prep_heads_kernel<false, false>);
+    hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kThreads), 0, stream, p,
+                       num_sequences, ws, chunk_start, records);
+  }
   hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(kThreads), 0, stream, p,
                      num_sequences, ws, chunk_start, records);
   return check_launch("ld_gdn_prefill (chunked)");

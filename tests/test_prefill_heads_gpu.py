@@ -47,19 +47,29 @@ def test_chunk_edges(gpu, heads):
     check(case)
 
 
-@pytest.mark.parametrize("lengths", [[64], [65], [64, 64, 64, 64], [65, 64, 64, 64],
-                                     [80, 33, 70, 81, 90]])
+@pytest.mark.parametrize("lengths", [[128], [129], [128, 128], [129, 128], [256] * 4,
+                                     [257, 256, 256, 256], [80, 33, 70, 81, 90]])
 def test_both_sides_of_the_rule(gpu, lengths):
-    """One prompt of 64 and of 65 tokens, four sequences of 64 on average and just above (128
-    pairs), five sequences (160 pairs)."""
+    """Up to 64 (sequence, head) pairs a mean of 128 tokens and just above, up to 128 pairs one
+    of 256 and just above, and 160 pairs."""
     announce(test="heads_rule", lengths=lengths)
     check(prefill_case(gpu, lengths, seed=len(lengths)))
 
 
+@pytest.mark.parametrize("heads,lengths", [((16, 48), [290, 353, 261]), ((16, 48), [256] * 3),
+                                           ((16, 48), [257, 256, 256]), ((32, 32), [1025, 1, 2, 3, 300])])
+def test_both_sides_of_the_record_rule(gpu, heads, lengths):
+    """A mean of up to 256 tokens, where a workgroup prepares its chunks itself (nine of them
+    here: three rounds of four), and above, where a launch ahead writes their records."""
+    announce(test="heads_records", heads=heads, lengths=lengths)
+    check(prefill_case(gpu, lengths, heads=heads, seed=sum(lengths), dt_dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("lengths", [[70, 33, 1, 0, 64, 90], [300, 270, 0, 290, 280, 500]])
 @pytest.mark.parametrize("what", ["qkv", "gate", "out"])
-def test_unaligned_rows_give_the_aligned_bits(gpu, what):
-    announce(test="heads_unaligned", what=what)
-    case = prefill_case(gpu, [70, 33, 1, 0, 64, 90], seed=3)
+def test_unaligned_rows_give_the_aligned_bits(gpu, what, lengths):
+    announce(test="heads_unaligned", what=what, lengths=lengths)
+    case = prefill_case(gpu, lengths, seed=3)
     pool0 = case["pool"].clone()
     run(case)
     torch.cuda.synchronize()
