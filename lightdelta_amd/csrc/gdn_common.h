@@ -141,15 +141,38 @@ inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
 int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequences,
                                         int64_t num_v_heads);
 // chunk_tokens: 64 or 32
-// *normed: whether `out` holds the final outputs (else the raw ones)
+// Which kernels the 32-token form runs: the whole-head ones (prefill_heads.hip: a workgroup per
+// (sequence, v-head)) or chunk_prep32_kernel and chunk_scan32_kernel (a head's rows over four
+// workgroups).  A chunk takes a lone workgroup of the first 3.2 us and of the second 2.3 us, but
+// with the chip full a (chunk, v-head) takes the first 17 ns and the second 30 ns; so it is
+// decided by how many heads' chains the batch keeps going beside its longest: heads x chunks /
+// longest chain, the number of (sequence, head) pairs if the prompts are equally long.  Over
+// short chains the launches and records that the first saves decide.
+struct HeadsRule {
+  int num_v_heads;
+  int short_chunks;   // whole heads up to this many chunks in the longest chain
+  int chains;         // or from this many chains
+  __host__ __device__ bool whole_heads(int64_t chunks, int64_t longest) const {
+    return longest <= short_chunks || chunks * num_v_heads > chains * longest;
+  }
+};
+
+// What a chunked prefill leaves in `out`: the final outputs (normed), or the raw ones unless
+// *form is set (null: raw).
+struct ChunkedOut {
+  bool normed = false;
+  const int32_t* form = nullptr;
+};
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
                            bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
-                           hipStream_t stream, bool* normed);
+                           hipStream_t stream, ChunkedOut* result);
 // The whole-head scan of 32-token chunks (prefill_heads.hip).  own: it prepares its chunks itself;
-// else a launch of its own does, into `records` records of kHeadRecordBytes at ws.
+// else a launch of its own does, into `records` records of kHeadRecordBytes at ws.  With `form`
+// these kernels return at once unless that device word is set.
 constexpr int64_t kHeadRecordBytes = 9728;
 int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float* ws,
-                       const int32_t* chunk_start, int records, bool dt_bf16, bool w_bf16,
+                       const int32_t* chunk_start, const int32_t* form, int records,
+                       bool dt_bf16, bool w_bf16,
                        hipStream_t stream);
 
 }  // namespace ld

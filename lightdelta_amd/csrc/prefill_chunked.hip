@@ -102,22 +102,31 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// Where both sides are launched, ahead of chunk_start in the workspace: chunk_start[-1] is the
+// decision (1: whole heads), chunk_start[-16 .. -9] the other scan's queues, one per XCD.
+constexpr int kXcds = 8;
+constexpr int kQueueAt = -15;   // from the decision
+
 // chunk_start[n] = sum over m < n of ceil(L_m / C) for n = 0 .. num_sequences: where the
 // chunks of sequence n begin in the global chunk order.  One workgroup, a block-wide scan per
-// 256 sequences.
+// 256 sequences.  With `form` also HeadsRule's decision there, and the scan's queues cleared.
 template <int C>
 __global__ __launch_bounds__(kThreads) void chunk_index_kernel(const int32_t* cu,
                                                                int num_sequences,
-                                                               int32_t* chunk_start) {
+                                                               int32_t* chunk_start,
+                                                               HeadsRule rule, int32_t* form) {
   __shared__ int32_t wave_total[kWaves];
+  __shared__ int32_t wave_longest[kWaves];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   if (tid == 0) chunk_start[0] = 0;
   int carry = 0;
+  int longest = 0;
   for (int base = 0; base < num_sequences; base += kThreads) {
     const int n = base + tid;
     int c = n < num_sequences ? (cu[n + 1] - cu[n] + C - 1) / C : 0;
+    longest = max(longest, c);
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const int up = __shfl_up(c, d);
@@ -135,6 +144,17 @@ __global__ __launch_bounds__(kThreads) void chunk_index_kernel(const int32_t* cu
     if (n < num_sequences) chunk_start[n + 1] = before + c;
     carry += total;
     __syncthreads();  // wave_total is rewritten by the next round
+  }
+  if (form == nullptr) return;
+  if (tid < kXcds) form[kQueueAt + tid] = 0;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) longest = max(longest, __shfl_xor(longest, d));
+  if (lane == 0) wave_longest[wave] = longest;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) longest = max(longest, wave_longest[w]);
+    *form = rule.whole_heads(carry, longest) ? 1 : 0;
   }
 }
 
@@ -667,13 +687,12 @@ __device__ __forceinline__ uint32_t prep32_tile(int index) {
 }
 
 template <bool DtBf16, bool Wide>
-__global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
-void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
-                         const int32_t* chunk_start, int records) {
+__device__ __forceinline__ void prep32_unit(const DecodeParams& p, int num_sequences, float* ws,
+                                            const int32_t* chunk_start, int records,
+                                            int64_t unit) {   // chunk * H + k-head
   using R = Rec32;
   constexpr int kCs = R::kC;
   constexpr int kTokens = kCs / (kPrep32Threads / 64);   // tokens normalised per wave
-  const int64_t unit = blockIdx.x;   // chunk * H + k-head
   const int g = static_cast<int>(unit / p.num_k_heads);
   if (g >= records) return;
   const int key_head = static_cast<int>(unit - static_cast<int64_t>(g) * p.num_k_heads);
@@ -962,6 +981,22 @@ void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
     }
     // the next v-head writes -A after its first barrier (every read of -A and T above is
     // behind one of this v-head's) and its gates went to the other buffer
+  }
+}
+
+// One workgroup per (chunk, k-head), or (Many) a grid that fits the chip and goes over them: with
+// `form` (the whole-head kernels' batch if it is set) a launch in vain then costs 2 us, where
+// 16,384 workgroups that return at once took 8.
+template <bool DtBf16, bool Wide, bool Many>
+__global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
+void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
+                         const int32_t* chunk_start, int records, const int32_t* form) {
+  if (form != nullptr && *form != 0) return;
+  const int64_t units = static_cast<int64_t>(records) * p.num_k_heads;
+  for (int64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+    prep32_unit<DtBf16, Wide>(p, num_sequences, ws, chunk_start, records, unit);
+    if (!Many) return;
+    __syncthreads();   // the LDS tiles are rewritten
   }
 }
 
@@ -1467,16 +1502,14 @@ __device__ __forceinline__ void load_output32(Scan32Output& o, __amdgpu_buffer_r
 // The products with S and with V_new ck on the bf16 matrix cores, each as three products
 // against split4's parts (fp32-exact operands, fp32 sums, 80 VGPRs).  (Prompts of one
 // chunk once kept fp32 products, before the splits took one instruction per remainder.)
-__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(6)))
-void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
-                         const int32_t* chunk_start, int records) {
+__device__ __forceinline__ void scan32_rows(const DecodeParams& p, int num_sequences, float* ws,
+                                            const int32_t* chunk_start, int records, int xcd,
+                                            int rank) {
   using R = Rec32;
   constexpr int kCs = R::kC;                 // 32 tokens per chunk
   constexpr int kRows = 32;                  // state rows per workgroup
   constexpr int kBlocks = kDim / kRows;
   // XCD-aware ids as in chunk_scan_kernel: the 4 row blocks of one (sequence, head) on one XCD
-  const int xcd = blockIdx.x & 7;
-  const int rank = blockIdx.x >> 3;
   const int pair = (rank / kBlocks) * 8 + xcd;
   if (pair >= num_sequences * p.num_v_heads) return;
   const int seq = pair / p.num_v_heads;
@@ -1744,6 +1777,32 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
   }
 }
 
+// One workgroup per (pair, row block).  Many: a fixed grid whose workgroups take them from their
+// XCD's queue (see chunk_prep32_kernel; 65,536 workgroups that return at once took 25 us).  The
+// loop's registers cost it two of six waves a SIMD.
+template <bool Many>
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(Many ? 4 : 6)))
+void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
+                         const int32_t* chunk_start, int records, int32_t* form) {
+  if (form != nullptr && *form != 0) return;
+  const int xcd = blockIdx.x & (kXcds - 1);
+  int rank = blockIdx.x / kXcds;
+  if constexpr (!Many) {
+    scan32_rows(p, num_sequences, ws, chunk_start, records, xcd, rank);
+  } else {
+    __shared__ int taken;
+    const int ranks = (num_sequences * p.num_v_heads + kXcds - 1) / kXcds * (kDim / 32);
+    while (rank < ranks) {
+      if (threadIdx.x == 0)
+        taken = atomicAdd(form + kQueueAt + xcd, 1) + static_cast<int>(gridDim.x) / kXcds;
+      scan32_rows(p, num_sequences, ws, chunk_start, records, xcd, rank);
+      __syncthreads();   // (and the LDS tiles are rewritten)
+      rank = __builtin_amdgcn_readfirstlane(taken);
+      __syncthreads();
+    }
+  }
+}
+
 template <int C>
 int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
   return num_tokens / C + num_sequences;  // each sequence adds at most one partial chunk
@@ -1751,39 +1810,32 @@ int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
 
 // Workspace: the records, then chunk_start (num_sequences + 1 int32, rounded up to 256 B).
 // Sized for 64-token chunks, which covers 32-token ones: with S >= 1 sequences,
-// (T / 32 + S) R32 <= (2 (T / 64) + 1 + S) R32 <= (T / 64 + S) R64 as 2 R32 <= R64.
-static_assert(2 * Rec32::kSize <= kRecord && kHeadRecordBytes <= Rec32::kSize * 4,
+// (T / 32 + S) R32 <= (2 (T / 64) + 1 + S) R32 < (T / 64 + S) R64 as 2 R32 < R64; the word
+// ahead of chunk_start is the 32-token form's `form`.
+static_assert(2 * Rec32::kSize < kRecord && kHeadRecordBytes <= Rec32::kSize * 4,
               "32-token records fit the workspace");
 int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
 }
 
-// Which scan the 32-token form runs: chunk_heads_kernel (a whole head per workgroup, norm
-// fused) or chunk_scan32_kernel (a head's rows over four workgroups).  A chunk takes a lone
-// workgroup of the first 3.2 us and of the second 2.3 us, so with few (sequence, head) pairs
-// the second's chain is the shorter; from two chunks per CU on the first's throughput decides,
-// and for short prompts the launches it saves (us, first / second, at 32 v-heads: 1 x 128 25 /
-// 27, 1 x 192 35 / 31, 2 x 128 25 / 29, 2 x 256 43 / 39, 4 x 192 37 / 42, 4 x 256 46 / 48,
-// 4 x 320 56 / 54, 4 x 1024 144 / 137, 5 x 1024 137 / 181, 8 x 1024 162 / 258, 32 x 1024 586 /
-// 985).
-bool whole_heads(int64_t num_tokens, int64_t num_sequences, int64_t num_v_heads) {
-  const int64_t pairs = num_sequences * num_v_heads;
-  return pairs > 128 || num_tokens <= (pairs > 64 ? 256 : 128) * num_sequences;
-}
+// Prompts up to this mean length have their records prepared by the scan's own workgroups, which
+// saves the record launch and the records (us, with records / own: 1 x 64 26.5 / 19.7, 16 x 64
+// 41.9 / 31.9, 8 x 128 39.5 / 28.4, 8 x 256 53.2 / 49.4, 32 x 256 169 / 155, 1024 x 32 1266 /
+// 1196) but lengthens a chunk's step in its chain by 1 us (13 prompts up to 3000 tokens 265 / 338,
+// 8 x 1024 161 / 177).
+constexpr int64_t kOwnTokens = 256;
 
+// Of HeadsRule's two sides, where the host's numbers leave no choice only one is launched; else
+// both are, it is decided from the lengths on the device, and the other side's workgroups return
+// at once: 4 to 10 us of launches (us, row blocks / whole heads / so decided: 32 x 1024 985 / 586
+// / 590, 512 prompts of 8 to 56 994 / 631 / 641, 16 x 64 52 / 32 / 40, one of 4096 and 15 of 16
+// 277 / 430 / 284, one of 1000 and 30 of 40 108 / 162 / 112, 5 of 1 to 6000 179 / 272 / 184, 32
+// of 1 to 1000 206 / 179 / 191; one of 8192 and 511 of 20, by the Many kernels, 1025 / - / 1206).
+constexpr int64_t kManyGroups = 32768;   // of the scan: beyond them the Many kernels
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
                   bool w_bf16, float* ws, int32_t* chunk_start, hipStream_t stream,
-                  bool* normed) {
-  *normed = TT == 2 && whole_heads(num_tokens, num_sequences, p.num_v_heads);
-  // Short prompts' workgroups prepare their few chunks themselves: two launches fewer and no
-  // records in memory (us, with records / own: 1 x 64 26.5 / 19.7, 16 x 64 41.9 / 31.9, 8 x 128
-  // 39.5 / 28.4, 8 x 256 53.2 / 49.4, 32 x 256 169 / 155, 1024 x 32 1266 / 1196); over many
-  // chunks it lengthens the chain by 1 us a chunk (13 prompts up to 3000 tokens 265 / 338,
-  // 8 x 1024 161 / 177).
-  const bool own = num_tokens <= 256 * static_cast<int64_t>(num_sequences);
-  if (*normed && own)
-    return launch_chunk_heads(p, num_sequences, true, nullptr, nullptr, 0, dt_bf16, w_bf16, stream);
+                  ChunkedOut* result) {
   constexpr int kCt = TT == 2 ? Rec32::kC : kC;
   const int64_t chunks = max_chunks<kCt>(num_tokens, num_sequences);
   if (chunks > 0x7fffffff || p.num_v_heads > 65535)
@@ -1791,44 +1843,57 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   // one workgroup per (chunk, k-head)
   const int64_t prep_groups = chunks * p.num_k_heads;
   if (prep_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
-  const dim3 per_chunk(static_cast<uint32_t>(prep_groups));
-  hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
-                     num_sequences, chunk_start);
-  if (*normed)
-    return launch_chunk_heads(p, num_sequences, false, ws, chunk_start, static_cast<int>(chunks),
-                              dt_bf16, w_bf16, stream);
+  const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
+  int32_t* form = nullptr;
+  HeadsRule rule{};
+  if constexpr (TT == 2) {
+    rule.num_v_heads = p.num_v_heads;
+    const bool own = num_tokens <= kOwnTokens * num_sequences;
+    rule.short_chunks = !own ? 0 : pairs > 64 ? 8 : 4;
+    rule.chains = own ? 128 : 96;
+    // (the longest chain has at least the mean's length, and at most all the tokens'; up to 128
+    // pairs only prompts of nearly one length would gain: 4 x 1024 7 of 145 us)
+    const bool may = pairs > 128 || num_tokens <= rule.short_chunks * kCt * static_cast<int64_t>(num_sequences);
+    result->normed = (num_tokens + kCt - 1) / kCt <= rule.short_chunks || p.num_v_heads > rule.chains;
+    if (may && !result->normed) form = chunk_start - 1;   // (past the 32-token form's records)
+    if (!own || !result->normed)
+      hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
+                         num_sequences, chunk_start, rule, form);
+    if (result->normed || form != nullptr) {
+      const int rc = launch_chunk_heads(p, num_sequences, own, ws, chunk_start, form,
+                                        static_cast<int>(chunks), dt_bf16, w_bf16, stream);
+      if (rc != LD_OK || result->normed) return rc;
+    }
+    result->form = form;
+  } else {
+    hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
+                       num_sequences, chunk_start, rule, form);
+  }
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;
-#define LD_PREP_LAUNCH(K, D, W, N)                                                             \
-  hipLaunchKernelGGL((K<D, W>), per_chunk, dim3(N), 0, stream, p, num_sequences, ws,          \
-                     chunk_start, static_cast<int>(chunks))
-#define LD_PREP_LAUNCHES(K, N)                                                                 \
-  if (dt_bf16) {                                                                               \
-    if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, true, true, N);                                                        \
-    else                                                                                       \
-      LD_PREP_LAUNCH(K, true, false, N);                                                       \
-  } else {                                                                                     \
-    if (wide)                                                                                  \
-      LD_PREP_LAUNCH(K, false, true, N);                                                       \
-    else                                                                                       \
-      LD_PREP_LAUNCH(K, false, false, N);                                                      \
-  }
-   if constexpr (TT == 2) {
-    LD_PREP_LAUNCHES(chunk_prep32_kernel, kPrep32Threads)
-  } else {
-    LD_PREP_LAUNCHES(chunk_prep_kernel, kPrepThreads)
-  }
-#undef LD_PREP_LAUNCHES
-#undef LD_PREP_LAUNCH
-  const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
+#define LD_PREP(K, ...)                                                                        \
+  (dt_bf16 ? (wide ? K<true, true __VA_ARGS__> : K<true, false __VA_ARGS__>)                   \
+           : (wide ? K<false, true __VA_ARGS__> : K<false, false __VA_ARGS__>))
+#define LD_COMMA ,
   if constexpr (TT == 2) {
-    const int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
+    int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
     if (scan_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
-    hipLaunchKernelGGL(chunk_scan32_kernel, dim3(static_cast<uint32_t>(scan_groups)),
-                       dim3(kScanThreads), 0, stream, p, num_sequences, ws, chunk_start,
-                       static_cast<int>(chunks));
+    const bool many = form != nullptr && scan_groups > kManyGroups;
+    const int64_t prep_grid = many ? std::min<int64_t>(prep_groups, 1280) : prep_groups;   // 5 a CU
+    if (many) scan_groups = 1024;
+    const auto prep = many ? LD_PREP(chunk_prep32_kernel, LD_COMMA true)
+                           : LD_PREP(chunk_prep32_kernel, LD_COMMA false);
+    hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_grid)), dim3(kPrep32Threads), 0,
+                       stream, p, num_sequences, ws, chunk_start, static_cast<int>(chunks), form);
+    hipLaunchKernelGGL(many ? chunk_scan32_kernel<true> : chunk_scan32_kernel<false>,
+                       dim3(static_cast<uint32_t>(scan_groups)), dim3(kScanThreads), 0, stream, p,
+                       num_sequences, ws, chunk_start, static_cast<int>(chunks), form);
   } else {
+    const auto prep = LD_PREP(chunk_prep_kernel);
+    hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kPrepThreads), 0,
+                       stream, p, num_sequences, ws, chunk_start, static_cast<int>(chunks));
+#undef LD_COMMA
+#undef LD_PREP
     // two row tiles per workgroup once they still give 2 workgroups per CU
     const bool two_tiles = pairs * (kDim / 32) >= 512;
     const int64_t scan_groups = (pairs + 7) / 8 * 8 * (two_tiles ? kDim / 32 : kDim / 16);
@@ -1855,15 +1920,15 @@ int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequence
 
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
                            bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
-                           hipStream_t stream, bool* normed) {
+                           hipStream_t stream, ChunkedOut* result) {
   float* ws = static_cast<float*>(workspace);
   int32_t* chunk_start = reinterpret_cast<int32_t*>(
       static_cast<char*>(workspace) + records_bytes(num_tokens, num_sequences, p.num_v_heads));
   if (chunk_tokens == 32)
     return launch_chunks<2>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start,
-                            stream, normed);
+                            stream, result);
   return launch_chunks<4>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start, stream,
-                          normed);
+                          result);
 }
 
 }  // namespace ld

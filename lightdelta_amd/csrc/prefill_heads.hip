@@ -32,7 +32,7 @@
 // GHz (a large bf16 GEMM reaches 1.17), 438 us, where chunk_scan32_kernel and the norm pass
 // took 820 us: with a head's rows over four workgroups every wave re-read S's planes from LDS
 // and the raw outputs crossed HBM twice more.  The whole prefill, with the prep
-// below, went from 985 to 586 us there, 257 to 164 us at 8 x 1024, 1,710 to 1,264 us at
+// below, went from 985 to 585 us there, 257 to 169 us at 8 x 1024, 1,710 to 1,195 us at
 // 1024 x 32.  Products and vector work
 // are laid out by hand, slot by slot: as the compiler scheduled the same code, 32 x 1024 took
 // 685 us.
@@ -558,7 +558,8 @@ __device__ __forceinline__ void prep_head(const PrepTiles& x, const PrepGates& i
 template <bool DtBf16, bool Wide>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
-                             const int32_t* chunk_start, int records) {
+                             const int32_t* chunk_start, const int32_t* form, int records) {
+  if (form != nullptr && *form == 0) return;
   __shared__ __attribute__((aligned(16))) PrepScratch scratch[kWaves];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
@@ -594,7 +595,8 @@ void chunk_prep_heads_kernel(const DecodeParams p, int num_sequences, float* ws,
 template <bool Own, bool DtBf16, bool WBf16, bool Wide>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws,
-                        const int32_t* chunk_start, int records) {
+                        const int32_t* chunk_start, const int32_t* form, int records) {
+  if (form != nullptr && *form == 0) return;   // (another form's batch)
   using R = Record;
   // Workgroups go to the 8 XCDs round-robin by id; the v-heads of one (sequence, k-head) read
   // the same q and k, so they are given ids on one XCD.
@@ -1074,8 +1076,8 @@ void chunk_heads_kernel(const DecodeParams p, int num_sequences, const float* ws
 }  // namespace
 
 int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float* ws,
-                       const int32_t* chunk_start, int records, bool dt_bf16, bool w_bf16,
-                       hipStream_t stream) {
+                       const int32_t* chunk_start, const int32_t* form, int records,
+                       bool dt_bf16, bool w_bf16, hipStream_t stream) {
   const int64_t units = static_cast<int64_t>(num_sequences) * p.num_k_heads;
   const int64_t groups = (units + 7) / 8 * 8 * p.group;
   const int64_t prep_groups = (static_cast<int64_t>(records) * p.num_k_heads + kWaves - 1) / kWaves;
@@ -1095,10 +1097,10 @@ int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float
     const auto prep = dt_bf16 ? (wide_qkv ? chunk_prep_heads_kernel<true, true> : chunk_prep_heads_kernel<true, false>)
                               : (wide_qkv ? chunk_prep_heads_kernel<false, true> : chunk_prep_heads_kernel<false, false>);
     hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kThreads), 0, stream, p,
-                       num_sequences, ws, chunk_start, records);
+                       num_sequences, ws, chunk_start, form, records);
   }
   hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups)), dim3(kThreads), 0, stream, p,
-                     num_sequences, ws, chunk_start, records);
+                     num_sequences, ws, chunk_start, form, records);
   return check_launch("ld_gdn_prefill (chunked)");
 }
 

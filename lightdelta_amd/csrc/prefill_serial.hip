@@ -352,55 +352,60 @@ constexpr int kNormItems = 8;
 
 template <bool WBf16, bool Pairs>
 __global__ __launch_bounds__(kThreads) void prefill_norm_kernel(const DecodeParams p,
-                                                                int num_sequences) {
+                                                                int num_sequences,
+                                                                const int32_t* form) {
+  if (form != nullptr && *form != 0) return;   // (normed by the whole-head kernels)
   const int lane = threadIdx.x & 63;
-  const int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6)) *
-                        kNormItems;
   const int64_t lo = static_cast<int64_t>(p.cu[0]) * p.num_v_heads;
   const int64_t hi = static_cast<int64_t>(p.cu[num_sequences]) * p.num_v_heads;
-  if (first >= hi || first + kNormItems <= lo) return;  // no row of this wave (or none at all)
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves * kNormItems;
+  int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6)) * kNormItems;
+  while (first + kNormItems <= lo) first += stride;   // no row of this wave
+  if (first >= hi) return;
   float w[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) w[e] = load_param(p.norm_weight, 2 * lane + e, WBf16);
-  uint32_t raw_bits[kNormItems], gate_bits[kNormItems];
+  for (; first < hi; first += stride) {
+    uint32_t raw_bits[kNormItems], gate_bits[kNormItems];
 #pragma unroll
-  for (int n = 0; n < kNormItems; ++n) {
-    const int64_t item = min(max(first + n, lo), hi - 1);  // in range; unused ones not stored
-    const int64_t token = item / p.num_v_heads;
-    const int head = static_cast<int>(item - token * p.num_v_heads);
-    const uint16_t* row = p.out + item * kDim + 2 * lane;
-    const uint16_t* grow = p.gate + token * p.gate_row + head * kDim + 2 * lane;
-    if (Pairs) {
-      raw_bits[n] = *reinterpret_cast<const uint32_t*>(row);
-      gate_bits[n] = *reinterpret_cast<const uint32_t*>(grow);
-    } else {
-      raw_bits[n] = row[0] | (static_cast<uint32_t>(row[1]) << 16);
-      gate_bits[n] = grow[0] | (static_cast<uint32_t>(grow[1]) << 16);
-    }
-  }
-#pragma unroll
-  for (int n = 0; n < kNormItems; ++n) {
-    const int64_t item = first + n;
-    float raw[2], gate[2];
-    raw[0] = bf16_to_f32(static_cast<uint16_t>(raw_bits[n]));
-    raw[1] = bf16_to_f32(static_cast<uint16_t>(raw_bits[n] >> 16));
-    gate[0] = bf16_to_f32(static_cast<uint16_t>(gate_bits[n]));
-    gate[1] = bf16_to_f32(static_cast<uint16_t>(gate_bits[n] >> 16));
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) ss = fmaf(raw[e], raw[e], ss);
-    ss = wave_sum(ss);
-    const float rstd = fast_rsqrt(ss / static_cast<float>(kDim) + p.eps);
-    uint16_t y[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) y[e] = f32_to_bf16(((raw[e] * rstd) * w[e]) * silu(gate[e]));
-    if (item >= lo && item < hi) {
-      uint16_t* row = p.out + item * kDim + 2 * lane;
+    for (int n = 0; n < kNormItems; ++n) {
+      const int64_t item = min(max(first + n, lo), hi - 1);  // in range; unused ones not stored
+      const int64_t token = item / p.num_v_heads;
+      const int head = static_cast<int>(item - token * p.num_v_heads);
+      const uint16_t* row = p.out + item * kDim + 2 * lane;
+      const uint16_t* grow = p.gate + token * p.gate_row + head * kDim + 2 * lane;
       if (Pairs) {
-        *reinterpret_cast<uint32_t*>(row) = y[0] | (static_cast<uint32_t>(y[1]) << 16);
+        raw_bits[n] = *reinterpret_cast<const uint32_t*>(row);
+        gate_bits[n] = *reinterpret_cast<const uint32_t*>(grow);
       } else {
-        row[0] = y[0];
-        row[1] = y[1];
+        raw_bits[n] = row[0] | (static_cast<uint32_t>(row[1]) << 16);
+        gate_bits[n] = grow[0] | (static_cast<uint32_t>(grow[1]) << 16);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < kNormItems; ++n) {
+      const int64_t item = first + n;
+      float raw[2], gate[2];
+      raw[0] = bf16_to_f32(static_cast<uint16_t>(raw_bits[n]));
+      raw[1] = bf16_to_f32(static_cast<uint16_t>(raw_bits[n] >> 16));
+      gate[0] = bf16_to_f32(static_cast<uint16_t>(gate_bits[n]));
+      gate[1] = bf16_to_f32(static_cast<uint16_t>(gate_bits[n] >> 16));
+      float ss = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) ss = fmaf(raw[e], raw[e], ss);
+      ss = wave_sum(ss);
+      const float rstd = fast_rsqrt(ss / static_cast<float>(kDim) + p.eps);
+      uint16_t y[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) y[e] = f32_to_bf16(((raw[e] * rstd) * w[e]) * silu(gate[e]));
+      if (item >= lo && item < hi) {
+        uint16_t* row = p.out + item * kDim + 2 * lane;
+        if (Pairs) {
+          *reinterpret_cast<uint32_t*>(row) = y[0] | (static_cast<uint32_t>(y[1]) << 16);
+        } else {
+          row[0] = y[0];
+          row[1] = y[1];
+        }
       }
     }
   }
@@ -413,57 +418,62 @@ __global__ __launch_bounds__(kThreads) void prefill_norm_kernel(const DecodePara
 // wave_sum's remaining levels), so the results are those of prefill_norm_kernel, bit for bit.
 template <bool WBf16>
 __global__ __launch_bounds__(kThreads) void prefill_norm_wide_kernel(const DecodeParams p,
-                                                                     int num_sequences) {
+                                                                     int num_sequences,
+                                                                const int32_t* form) {
+  if (form != nullptr && *form != 0) return;   // (normed by the whole-head kernels)
   const int lane = threadIdx.x & 63;
   const int r = lane >> 4;
   const int c = lane & 15;
-  const int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6)) *
-                        kNormItems;
   const int64_t lo = static_cast<int64_t>(p.cu[0]) * p.num_v_heads;
   const int64_t hi = static_cast<int64_t>(p.cu[num_sequences]) * p.num_v_heads;
-  if (first >= hi || first + kNormItems <= lo) return;  // no row of this wave (or none at all)
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves * kNormItems;
+  int64_t first = (static_cast<int64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6)) * kNormItems;
+  while (first + kNormItems <= lo) first += stride;   // no row of this wave
+  if (first >= hi) return;
   constexpr int kLoads = kNormItems / 4;
   float w[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) w[e] = load_param(p.norm_weight, 8 * c + e, WBf16);
-  u32x4 raw_bits[kLoads], gate_bits[kLoads];
+  for (; first < hi; first += stride) {
+    u32x4 raw_bits[kLoads], gate_bits[kLoads];
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) {
-    const int64_t item = min(max(first + 4 * j + r, lo), hi - 1);  // in range; unused ones not stored
-    const int64_t token = item / p.num_v_heads;
-    const int head = static_cast<int>(item - token * p.num_v_heads);
-    raw_bits[j] = *reinterpret_cast<const u32x4*>(p.out + item * kDim + 8 * c);
-    gate_bits[j] = *reinterpret_cast<const u32x4*>(p.gate + token * p.gate_row + head * kDim + 8 * c);
-  }
-#pragma unroll
-  for (int j = 0; j < kLoads; ++j) {
-    const int64_t item = first + 4 * j + r;
-    float raw[8], gate[8];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      raw[2 * m] = __builtin_bit_cast(float, raw_bits[j][m] << 16);
-      raw[2 * m + 1] = __builtin_bit_cast(float, raw_bits[j][m] & 0xffff0000u);
-      gate[2 * m] = __builtin_bit_cast(float, gate_bits[j][m] << 16);
-      gate[2 * m + 1] = __builtin_bit_cast(float, gate_bits[j][m] & 0xffff0000u);
+    for (int j = 0; j < kLoads; ++j) {
+      const int64_t item = min(max(first + 4 * j + r, lo), hi - 1);  // in range; unused ones not stored
+      const int64_t token = item / p.num_v_heads;
+      const int head = static_cast<int>(item - token * p.num_v_heads);
+      raw_bits[j] = *reinterpret_cast<const u32x4*>(p.out + item * kDim + 8 * c);
+      gate_bits[j] = *reinterpret_cast<const u32x4*>(p.gate + token * p.gate_row + head * kDim + 8 * c);
     }
-    float pq[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) pq[m] = fmaf(raw[2 * m + 1], raw[2 * m + 1], raw[2 * m] * raw[2 * m]);
-    float ss = (pq[0] + pq[1]) + (pq[2] + pq[3]);
-    ss += dpp<kDppQuadXor1>(ss);
-    ss += dpp<kDppQuadXor2>(ss);
-    ss += dpp<kDppRowHalfMirror>(ss);
-    ss += dpp<kDppRowMirror>(ss);
-    const float rstd = fast_rsqrt(ss / static_cast<float>(kDim) + p.eps);
-    uint32_t y[4];
+    for (int j = 0; j < kLoads; ++j) {
+      const int64_t item = first + 4 * j + r;
+      float raw[8], gate[8];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const uint16_t y0 = f32_to_bf16(((raw[2 * m] * rstd) * w[2 * m]) * silu(gate[2 * m]));
-      const uint16_t y1 = f32_to_bf16(((raw[2 * m + 1] * rstd) * w[2 * m + 1]) * silu(gate[2 * m + 1]));
-      y[m] = y0 | (static_cast<uint32_t>(y1) << 16);
+      for (int m = 0; m < 4; ++m) {
+        raw[2 * m] = __builtin_bit_cast(float, raw_bits[j][m] << 16);
+        raw[2 * m + 1] = __builtin_bit_cast(float, raw_bits[j][m] & 0xffff0000u);
+        gate[2 * m] = __builtin_bit_cast(float, gate_bits[j][m] << 16);
+        gate[2 * m + 1] = __builtin_bit_cast(float, gate_bits[j][m] & 0xffff0000u);
+      }
+      float pq[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) pq[m] = fmaf(raw[2 * m + 1], raw[2 * m + 1], raw[2 * m] * raw[2 * m]);
+      float ss = (pq[0] + pq[1]) + (pq[2] + pq[3]);
+      ss += dpp<kDppQuadXor1>(ss);
+      ss += dpp<kDppQuadXor2>(ss);
+      ss += dpp<kDppRowHalfMirror>(ss);
+      ss += dpp<kDppRowMirror>(ss);
+      const float rstd = fast_rsqrt(ss / static_cast<float>(kDim) + p.eps);
+      uint32_t y[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const uint16_t y0 = f32_to_bf16(((raw[2 * m] * rstd) * w[2 * m]) * silu(gate[2 * m]));
+        const uint16_t y1 = f32_to_bf16(((raw[2 * m + 1] * rstd) * w[2 * m + 1]) * silu(gate[2 * m + 1]));
+        y[m] = y0 | (static_cast<uint32_t>(y1) << 16);
+      }
+      if (item >= lo && item < hi)
+        *reinterpret_cast<u32x4*>(p.out + item * kDim + 8 * c) = u32x4{y[0], y[1], y[2], y[3]};
     }
-    if (item >= lo && item < hi)
-      *reinterpret_cast<u32x4*>(p.out + item * kDim + 8 * c) = u32x4{y[0], y[1], y[2], y[3]};
   }
 }
 
@@ -533,11 +543,11 @@ int prefill(const ld_gdn_prefill_args& a, void* workspace, int64_t workspace_byt
           ? prefill_auto_chunk_tokens(a.num_tokens, a.num_sequences, a.num_v_heads)
           : 0;
   const bool chunked = chunk_tokens != 0;
+  ChunkedOut out;
   if (chunked) {
-    bool normed = false;
     const int rc = launch_prefill_chunked(p, a.num_sequences, a.num_tokens, dt_bf16, w_bf16,
-                                          chunk_tokens, workspace, s, &normed);
-    if (rc != LD_OK || normed) return rc;
+                                          chunk_tokens, workspace, s, &out);
+    if (rc != LD_OK || out.normed) return rc;
   }
   // Token-serial: split a head's rows over more workgroups when (sequence, head) tiles alone
   // would leave the GPU short of work (1024 tiles fill 256 CUs at 4 per CU).
@@ -566,16 +576,18 @@ int prefill(const ld_gdn_prefill_args& a, void* workspace, int64_t workspace_byt
     const int64_t items = a.num_tokens * static_cast<int64_t>(a.num_v_heads);
     if (items > 0) {
       const int64_t per_block = static_cast<int64_t>(kWaves) * kNormItems;
-      const uint32_t norm_grid = static_cast<uint32_t>((items + per_block - 1) / per_block);
+      // (few workgroups where they may find the rows normed already)
+      const uint32_t norm_grid = static_cast<uint32_t>(
+          std::min<int64_t>((items + per_block - 1) / per_block, out.form != nullptr ? 2048 : 0x7fffffff));
       const bool pairs = (reinterpret_cast<uintptr_t>(a.gate) & 3) == 0 && (a.gate_row_stride & 1) == 0;
       const bool wide = (reinterpret_cast<uintptr_t>(a.gate) & 15) == 0 && (a.gate_row_stride & 7) == 0 &&
                         (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
 #define LD_NORM_LAUNCH(W, P)                                                                  \
   hipLaunchKernelGGL((prefill_norm_kernel<W, P>), dim3(norm_grid), dim3(kThreads), 0, s, p,  \
-                     a.num_sequences)
+                     a.num_sequences, out.form)
       if (wide) {
         hipLaunchKernelGGL(w_bf16 ? prefill_norm_wide_kernel<true> : prefill_norm_wide_kernel<false>,
-                           dim3(norm_grid), dim3(kThreads), 0, s, p, a.num_sequences);
+                           dim3(norm_grid), dim3(kThreads), 0, s, p, a.num_sequences, out.form);
       } else if (w_bf16) {
         if (pairs) LD_NORM_LAUNCH(true, true); else LD_NORM_LAUNCH(true, false);
       } else {

@@ -48,21 +48,43 @@ def test_chunk_edges(gpu, heads):
 
 
 @pytest.mark.parametrize("lengths", [[128], [129], [128, 128], [129, 128], [256] * 4,
-                                     [257, 256, 256, 256], [80, 33, 70, 81, 90]])
+                                     [257, 256, 256, 256], [80, 33, 70, 81, 90],
+                                     [330, 40, 10, 1, 70], [300, 256, 280, 270, 256]])
 def test_both_sides_of_the_rule(gpu, lengths):
-    """Up to 64 (sequence, head) pairs a mean of 128 tokens and just above, up to 128 pairs one
-    of 256 and just above, and 160 pairs."""
+    """The longest prompt at the limits of the short chains (up to 64 and to 128 (sequence, head)
+    pairs), 160 pairs, and batches that are decided on the device: a long prompt among short
+    ones, and equal ones."""
     announce(test="heads_rule", lengths=lengths)
     check(prefill_case(gpu, lengths, seed=len(lengths)))
 
 
 @pytest.mark.parametrize("heads,lengths", [((16, 48), [290, 353, 261]), ((16, 48), [256] * 3),
-                                           ((16, 48), [257, 256, 256]), ((32, 32), [1025, 1, 2, 3, 300])])
+                                           ((16, 32), [270, 250, 250, 250, 250])])
 def test_both_sides_of_the_record_rule(gpu, heads, lengths):
     """A mean of up to 256 tokens, where a workgroup prepares its chunks itself (nine of them
     here: three rounds of four), and above, where a launch ahead writes their records."""
     announce(test="heads_records", heads=heads, lengths=lengths)
     check(prefill_case(gpu, lengths, heads=heads, seed=sum(lengths), dt_dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("lengths", [[290, 1, 0, 70, 33] + [0] * 254 + [40], [3, 0, 1, 34] * 65])
+def test_many_sequences(gpu, lengths):
+    """Over 8,192 (sequence, head) pairs the row-block scan takes them from queues: a batch for it
+    (one long prompt) and one for the whole-head kernels, each replayed from a graph too."""
+    announce(test="heads_many", sequences=len(lengths))
+    case = prefill_case(gpu, lengths, seed=7)
+    pool0 = case["pool"].clone()
+    check(case)
+    out, pool = case["out"].clone(), case["pool"].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(case)
+    for _ in range(3):
+        case["pool"].copy_(pool0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(case["out"], out)
+        assert torch.equal(case["pool"], pool)
 
 
 @pytest.mark.parametrize("lengths", [[70, 33, 1, 0, 64, 90], [300, 270, 0, 290, 280, 500]])
