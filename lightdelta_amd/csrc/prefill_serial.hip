@@ -28,12 +28,19 @@ namespace {
 
 constexpr int kPrefillGroup = 4;
 
+// State tiles that the Infinity Cache (256 MB) holds.  Up to them plain loads and stores are the
+// faster where a call meets the states it left there (us, plain / non-temporal system-scope, 32
+// v-heads: 64 x 3 tokens 46 / 52, 96 x 3 67 / 77, 128 x 3 97 / 101); beyond, the others (160 x 3
+// 130 / 126, 200 x 3 177 / 155, 200 x 1..20 206 / 193, 1024 x 8 909 / 835).
+constexpr int64_t kCachedTiles = 4096;
+
 // One workgroup per (sequence, v-head), wave w holding rows 32w .. 32w + 31.  Tokens go in
 // groups of 4: before the group's barrier, wave w stages token w of the next group (q^ and
 // k^ in the lane layout, decay, beta: stage_token) into double-buffered LDS, and every wave
 // reads a token's staging from there, so each token is staged once per workgroup and off
-// the per-token chain.  A wave's v values come one token ahead.
-template <bool DtBf16, bool WBf16>
+// the per-token chain.  A wave's v values come one token ahead.  Pol: cache policy of the state's
+// loads and stores.
+template <bool DtBf16, bool WBf16, int Pol>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void gdn_prefill_kernel(const DecodeParams args) {
   constexpr int kWaveRows = 32;    // state rows per wave
@@ -82,7 +89,7 @@ void gdn_prefill_kernel(const DecodeParams args) {
         p.state + static_cast<int64_t>(slot) * p.state_slot + head_offset);
 #pragma unroll
     for (int j = 0; j < kTilePieces; ++j)
-      s[j] = *reinterpret_cast<const f32x4*>(src_tile + (lane_bytes + tile_piece_bytes(j)));
+      s[j] = load_tile_piece<Pol>(src_tile, lane_bytes + tile_piece_bytes(j));
   } else {
 #pragma unroll
     for (int j = 0; j < kTilePieces; ++j) s[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -212,9 +219,10 @@ void gdn_prefill_kernel(const DecodeParams args) {
   if (slot > 0) {  // the state after the last token (the initial one for an empty sequence)
     char* dst_tile = reinterpret_cast<char*>(p.state + static_cast<int64_t>(slot) * p.state_slot +
                                              head_offset);
+    TileStore<Pol> dst;
+    dst.set(dst_tile, true, nullptr);
 #pragma unroll
-    for (int j = 0; j < kTilePieces; ++j)
-      *reinterpret_cast<f32x4*>(dst_tile + (lane_bytes + tile_piece_bytes(j))) = s[j];
+    for (int j = 0; j < kTilePieces; ++j) dst.store(lane_bytes + tile_piece_bytes(j), s[j]);
   }
 }
 
@@ -553,11 +561,11 @@ int prefill(const ld_gdn_prefill_args& a, void* workspace, int64_t workspace_byt
   // would leave the GPU short of work (1024 tiles fill 256 CUs at 4 per CU).
   const int chunks = chunked ? 0 : (tiles >= 256 ? 4 : (tiles >= 128 ? 2 : 1));
   const uint32_t grid = chunks > 0 ? static_cast<uint32_t>(tiles * (4 / chunks)) : 0u;
-#define LD_PREFILL_LAUNCH()                                                                  \
-  hipLaunchKernelGGL(dt_bf16 ? (w_bf16 ? gdn_prefill_kernel<true, true>                      \
-                                       : gdn_prefill_kernel<true, false>)                    \
-                             : (w_bf16 ? gdn_prefill_kernel<false, true>                     \
-                                       : gdn_prefill_kernel<false, false>),                  \
+#define LD_PREFILL_LAUNCH(POL)                                                               \
+  hipLaunchKernelGGL(dt_bf16 ? (w_bf16 ? gdn_prefill_kernel<true, true, POL>                 \
+                                       : gdn_prefill_kernel<true, false, POL>)               \
+                             : (w_bf16 ? gdn_prefill_kernel<false, true, POL>                \
+                                       : gdn_prefill_kernel<false, false, POL>),             \
                      dim3(grid), dim3(kThreads), 0, s, p)
 #define LD_PREFILL_ROWS_LAUNCH(C)                                                            \
   hipLaunchKernelGGL(dt_bf16 ? (w_bf16 ? gdn_prefill_rows_kernel<true, true, C>              \
@@ -566,7 +574,10 @@ int prefill(const ld_gdn_prefill_args& a, void* workspace, int64_t workspace_byt
                                        : gdn_prefill_rows_kernel<false, false, C>),          \
                      dim3(grid), dim3(kThreads), 0, s, p)
   if (chunks == 4) {
-    LD_PREFILL_LAUNCH();
+    if (tiles > kCachedTiles)
+      LD_PREFILL_LAUNCH(kPolNTSys);
+    else
+      LD_PREFILL_LAUNCH(kPolPlain);
   } else {
     if (chunks == 2)
       LD_PREFILL_ROWS_LAUNCH(2);
