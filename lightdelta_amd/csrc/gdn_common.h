@@ -120,14 +120,13 @@ __device__ __forceinline__ float softplus(float x) {
 // on MI355X over 1 x 8 .. 4096 x 8 tokens at 32 v heads (ms, token-serial / 64-token
 // chunks / 32-token chunks):
 //   * token-serial below 17 tokens (1024 x 12: 1.30 / - / 1.51; 1024 x 16: 1.53-1.78 /
-//     3.03 / 1.50-1.55, where boxes of the pool disagree on the order; 1 x 16: 0.026 /
-//     0.032 / 0.030);
+//     3.03 / 1.50-1.55; 1 x 16: 0.026 / 0.032 / 0.030);
 //   * 64-token chunks for prompts of 512 tokens or more in fewer than 64 (sequence, head)
 //     pairs, where the chunk-by-chunk chain is the time and 64-token chunks halve it
 //     (1 x 4096: 2.74 / 0.201 / 0.279; 1 x 512: 0.357 / 0.051 / 0.056; 1 x 256: 0.183 /
 //     0.043 / 0.038; 2 x 2048, 64 pairs: 1.38 / 0.199 / 0.167);
 //   * 32-token chunks otherwise (1024 x 17: 1.63 / 3.06 / 1.53; 1024 x 32: 2.66 / 3.12 /
-//     1.72; 32 x 1024: 2.66 / 1.36 / 1.06; 1 x 64: 0.053 / 0.033 / 0.030).
+//     1.20; 32 x 1024: 2.66 / 1.36 / 0.59; 1 x 64: 0.053 / 0.033 / 0.020).
 // Returns the tokens per chunk (64 or 32), or 0 for the token-serial form.
 inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
                                      int64_t num_v_heads) {

@@ -51,9 +51,8 @@ def test_chunk_edges(gpu, heads):
                                      [257, 256, 256, 256], [80, 33, 70, 81, 90],
                                      [330, 40, 10, 1, 70], [300, 256, 280, 270, 256]])
 def test_both_sides_of_the_rule(gpu, lengths):
-    """The longest prompt at the limits of the short chains (up to 64 and to 128 (sequence, head)
-    pairs), 160 pairs, and batches that are decided on the device: a long prompt among short
-    ones, and equal ones."""
+    """Batches of up to 128 (sequence, head) pairs at the limits of the short chains, and 160 pairs,
+    decided on the device: short prompts, a long one among short ones, equal longer ones."""
     announce(test="heads_rule", lengths=lengths)
     check(prefill_case(gpu, lengths, seed=len(lengths)))
 
