@@ -4,6 +4,7 @@
 #pragma once
 
 #include "common.h"
+#include "prefill_rule.h"
 
 namespace ld {
 
@@ -140,22 +141,6 @@ inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
 int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequences,
                                         int64_t num_v_heads);
 // chunk_tokens: 64 or 32
-// Which kernels the 32-token form runs: the whole-head ones (prefill_heads.hip: a workgroup per
-// (sequence, v-head)) or chunk_prep32_kernel and chunk_scan32_kernel (a head's rows over four
-// workgroups).  A chunk takes a lone workgroup of the first 3.2 us and of the second 2.3 us, but
-// with the chip full a (chunk, v-head) takes the first 17 ns and the second 30 ns; so it is
-// decided by how many heads' chains the batch keeps going beside its longest: heads x chunks /
-// longest chain, the number of (sequence, head) pairs if the prompts are equally long.  Over
-// short chains the launches and records that the first saves decide.
-struct HeadsRule {
-  int num_v_heads;
-  int short_chunks;   // whole heads up to this many chunks in the longest chain
-  int chains;         // or from this many chains
-  __host__ __device__ bool whole_heads(int64_t chunks, int64_t longest) const {
-    return longest <= short_chunks || chunks * num_v_heads > chains * longest;
-  }
-};
-
 // What a chunked prefill leaves in `out`: the final outputs (normed), or the raw ones unless
 // *form is set (null: raw).
 struct ChunkedOut {

@@ -1818,19 +1818,6 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
 }
 
-// Prompts up to this mean length have their records prepared by the scan's own workgroups, which
-// saves the record launch and the records (us, with records / own: 1 x 64 26.5 / 19.7, 16 x 64
-// 41.9 / 31.9, 8 x 128 39.5 / 28.4, 8 x 256 53.2 / 49.4, 32 x 256 169 / 155, 1024 x 32 1266 /
-// 1196) but lengthens a chunk's step in its chain by 1 us (13 prompts up to 3000 tokens 265 / 338,
-// 8 x 1024 161 / 177).
-constexpr int64_t kOwnTokens = 256;
-
-// Of HeadsRule's two sides, where the host's numbers leave no choice only one is launched; else
-// both are, it is decided from the lengths on the device, and the other side's workgroups return
-// at once: 4 to 10 us of launches (us, row blocks / whole heads / so decided: 32 x 1024 985 / 586
-// / 590, 512 prompts of 8 to 56 994 / 631 / 641, 16 x 64 52 / 32 / 40, one of 4096 and 15 of 16
-// 277 / 430 / 284, one of 1000 and 30 of 40 108 / 162 / 112, 5 of 1 to 6000 179 / 272 / 184, 32
-// of 1 to 1000 206 / 179 / 191; one of 8192 and 511 of 20, by the Many kernels, 1025 / - / 1206).
 constexpr int64_t kManyGroups = 32768;   // of the scan: beyond them the Many kernels
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
@@ -1845,29 +1832,22 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   if (prep_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
   const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
   int32_t* form = nullptr;
-  HeadsRule rule{};
   if constexpr (TT == 2) {
-    rule.num_v_heads = p.num_v_heads;
-    const bool own = num_tokens <= kOwnTokens * num_sequences;
-    rule.short_chunks = !own ? 0 : pairs > 64 ? 8 : 4;
-    rule.chains = own ? 128 : 96;
-    // (up to 128 pairs the launches in vain would take what the decision gains: 3 x 100 34 / 34 us,
-    // 4 x 128 36 / 34, 4 x 1024 131 / 131)
-    const bool may = pairs > 128;
-    result->normed = (num_tokens + kCt - 1) / kCt <= rule.short_chunks || p.num_v_heads > rule.chains;
-    if (may && !result->normed) form = chunk_start - 1;   // (past the 32-token form's records)
-    if (!own || !result->normed)
+    const Plan32 plan = plan_chunks32(num_tokens, num_sequences, p.num_v_heads, p.gate_row);
+    result->normed = !plan.rows;
+    if (plan.heads && plan.rows) form = chunk_start - 1;   // (past the 32-token form's records)
+    if (!plan.own || plan.rows)
       hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
-                         num_sequences, chunk_start, rule, form);
-    if (result->normed || form != nullptr) {
-      const int rc = launch_chunk_heads(p, num_sequences, own, ws, chunk_start, form,
+                         num_sequences, chunk_start, plan.rule, form);
+    if (plan.heads) {
+      const int rc = launch_chunk_heads(p, num_sequences, plan.own, ws, chunk_start, form,
                                         static_cast<int>(chunks), dt_bf16, w_bf16, stream);
-      if (rc != LD_OK || result->normed) return rc;
+      if (rc != LD_OK || !plan.rows) return rc;
     }
     result->form = form;
   } else {
     hipLaunchKernelGGL(chunk_index_kernel<kCt>, dim3(1), dim3(kThreads), 0, stream, p.cu,
-                       num_sequences, chunk_start, rule, form);
+                       num_sequences, chunk_start, HeadsRule{}, form);
   }
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;

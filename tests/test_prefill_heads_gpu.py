@@ -11,6 +11,7 @@ import torch
 from lightdelta_amd import ops
 from oracle.decode import expected_prefill
 from tests.parity import assert_bf16_outputs, assert_states
+from tests.prefill_rule import side
 from tests.test_prefill_gpu import PREFILL, announce, prefill_case, run
 
 pytestmark = pytest.mark.gpu
@@ -118,4 +119,19 @@ def test_rows_of_one_shared_token(gpu):
     n = case["qkv"].shape[0]
     case["qkv"] = case["qkv"][:1].expand(n, -1)
     case["gate"] = case["gate"][:1].expand(n, -1, -1)
+    check(case)
+
+
+@pytest.mark.parametrize("row", [34_636_828, 34_636_829, 69_273_700])
+def test_far_apart_gate_rows(gpu, row):
+    """Gate rows at the largest stride whose offsets within a chunk fit 31 bits (whole heads), one
+    element farther apart, and so far that 32 bits would wrap (row blocks and the norm pass)."""
+    lengths = [33]
+    assert side(lengths, 32, row) == ("own" if row == 34_636_828 else "rows")
+    announce(test="heads_far_gate_rows", row=row)
+    case = prefill_case(gpu, lengths, seed=5)
+    far = torch.empty(32 * row + 4096, dtype=torch.bfloat16, device=gpu)
+    far = far.as_strided((33, 32, 128), (row, 128, 1))
+    far.copy_(case["gate"])
+    case["gate"] = far
     check(case)
