@@ -1821,8 +1821,8 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
 constexpr int64_t kManyGroups = 32768;   // of the scan: beyond them the Many kernels
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
-                  bool w_bf16, float* ws, int32_t* chunk_start, hipStream_t stream,
-                  ChunkedOut* result) {
+                  bool w_bf16, const Plan32& plan, float* ws, int32_t* chunk_start,
+                  hipStream_t stream, ChunkedOut* result) {
   constexpr int kCt = TT == 2 ? Rec32::kC : kC;
   const int64_t chunks = max_chunks<kCt>(num_tokens, num_sequences);
   if (chunks > 0x7fffffff || p.num_v_heads > 65535)
@@ -1833,7 +1833,6 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   const int64_t pairs = static_cast<int64_t>(num_sequences) * p.num_v_heads;
   int32_t* form = nullptr;
   if constexpr (TT == 2) {
-    const Plan32 plan = plan_chunks32(num_tokens, num_sequences, p.num_v_heads, p.gate_row);
     result->normed = !plan.rows;
     if (plan.heads && plan.rows) form = chunk_start - 1;   // (past the 32-token form's records)
     if (!plan.own || plan.rows)
@@ -1904,11 +1903,13 @@ int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num
   float* ws = static_cast<float*>(workspace);
   int32_t* chunk_start = reinterpret_cast<int32_t*>(
       static_cast<char*>(workspace) + records_bytes(num_tokens, num_sequences, p.num_v_heads));
-  if (chunk_tokens == 32)
-    return launch_chunks<2>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start,
+  const Plan32 plan = plan_chunks32(num_tokens, num_sequences, p.num_v_heads, p.gate_row);
+  const int64_t qkv_width = static_cast<int64_t>(2 * p.num_k_heads + p.num_v_heads) * kDim;
+  if (chunk_tokens == 32 && reads_qkv32(plan, p.qkv_row, qkv_width))
+    return launch_chunks<2>(p, num_sequences, num_tokens, dt_bf16, w_bf16, plan, ws, chunk_start,
                             stream, result);
-  return launch_chunks<4>(p, num_sequences, num_tokens, dt_bf16, w_bf16, ws, chunk_start, stream,
-                          result);
+  return launch_chunks<4>(p, num_sequences, num_tokens, dt_bf16, w_bf16, plan, ws, chunk_start,
+                          stream, result);
 }
 
 }  // namespace ld

@@ -30,10 +30,11 @@ struct HeadsRule {
 // 8 x 1024 161 / 177).
 constexpr int64_t kOwnTokens = 256;
 
-// Whether a chunk's 32 rows (`used` elements of 2 bytes, `row` elements apart) lie within the 31
-// bits that offsets from its first row have.
+// Whether a chunk's 32 rows (`used` elements of 2 bytes, `row` elements apart), and the row
+// after them, begin within the 31 bits that offsets from its first row and sizes of resources
+// over them have.
 constexpr bool chunk_rows_fit(int64_t row, int64_t used) {
-  return row >= 0 && row <= (0x7fffffff / 2 - used) / 31;
+  return row >= 0 && row <= (0x7fffffff / 2 - used) / 32;
 }
 
 struct Plan32 {
@@ -67,6 +68,14 @@ constexpr Plan32 plan_chunks32(int64_t num_tokens, int64_t num_sequences, int nu
   // 4 x 128 36 / 34, 4 x 1024 131 / 131)
   plan.heads = !plan.rows || pairs > 128;
   return plan;
+}
+
+// Whether these kernels read qkv with such rows rightly; if not, the 64-token form does, whose
+// preparation alone reads qkv, by 64-bit addresses.  The row-block scan's reads of v end at
+// `rows` row strides from the chunk's start: short of the last rows where rows overlap (a row
+// expanded over the tokens).
+constexpr bool reads_qkv32(const Plan32& plan, int64_t qkv_row, int64_t qkv_width) {
+  return chunk_rows_fit(qkv_row, qkv_width) && (!plan.rows || qkv_row >= qkv_width);
 }
 
 }  // namespace ld

@@ -18,6 +18,10 @@ extern "C" int plan(int64_t tokens, int64_t sequences, int heads, int64_t gate_r
   const ld::Plan32 p = ld::plan_chunks32(tokens, sequences, heads, gate_row);
   return (p.own ? 1 : 0) | (p.heads ? 2 : 0) | (p.rows ? 4 : 0);
 }
+extern "C" int reads_qkv(int64_t tokens, int64_t sequences, int heads, int64_t gate_row,
+                         int64_t qkv_row, int64_t qkv_width) {
+  return ld::reads_qkv32(ld::plan_chunks32(tokens, sequences, heads, gate_row), qkv_row, qkv_width);
+}
 extern "C" int whole_heads(int64_t tokens, int64_t sequences, int heads, int64_t gate_row,
                            int64_t chunks, int64_t longest) {
   return ld::plan_chunks32(tokens, sequences, heads, gate_row).rule.whole_heads(chunks, longest);
@@ -36,6 +40,7 @@ def _library():
         lib = ctypes.CDLL(str(built))
     i64 = ctypes.c_int64
     lib.plan.argtypes = [i64, i64, ctypes.c_int, i64]
+    lib.reads_qkv.argtypes = [i64, i64, ctypes.c_int, i64, i64, i64]
     lib.whole_heads.argtypes = [i64, i64, ctypes.c_int, i64, i64, i64]
     return lib
 
@@ -46,6 +51,12 @@ def plan(lengths, num_v_heads, gate_row=None):
     row = 128 * num_v_heads if gate_row is None else gate_row
     bits = _library().plan(sum(lengths), len(lengths), num_v_heads, row)
     return bool(bits & 1), bool(bits & 2), bool(bits & 4)
+
+
+def reads_qkv(lengths, num_v_heads, qkv_row, qkv_width):
+    """False: the 64-token form runs instead."""
+    return bool(_library().reads_qkv(sum(lengths), len(lengths), num_v_heads, 128 * num_v_heads,
+                                     qkv_row, qkv_width))
 
 
 def side(lengths, num_v_heads, gate_row=None):

@@ -11,7 +11,7 @@ import torch
 from lightdelta_amd import ops
 from oracle.decode import expected_prefill
 from tests.parity import assert_bf16_outputs, assert_states
-from tests.prefill_rule import side
+from tests.prefill_rule import reads_qkv, side
 from tests.test_prefill_gpu import PREFILL, announce, prefill_case, run
 
 pytestmark = pytest.mark.gpu
@@ -122,16 +122,44 @@ def test_rows_of_one_shared_token(gpu):
     check(case)
 
 
-@pytest.mark.parametrize("row", [34_636_828, 34_636_829, 69_273_700])
+@pytest.mark.parametrize("row", [33_554_427, 33_554_428, 69_273_700])
 def test_far_apart_gate_rows(gpu, row):
     """Gate rows at the largest stride whose offsets within a chunk fit 31 bits (whole heads), one
     element farther apart, and so far that 32 bits would wrap (row blocks and the norm pass)."""
     lengths = [33]
-    assert side(lengths, 32, row) == ("own" if row == 34_636_828 else "rows")
+    assert side(lengths, 32, row) == ("own" if row == 33_554_427 else "rows")
     announce(test="heads_far_gate_rows", row=row)
     case = prefill_case(gpu, lengths, seed=5)
     far = torch.empty(32 * row + 4096, dtype=torch.bfloat16, device=gpu)
     far = far.as_strided((33, 32, 128), (row, 128, 1))
     far.copy_(case["gate"])
     case["gate"] = far
+    check(case)
+
+
+@pytest.mark.parametrize("lengths", [[130], [300, 40, 1], [330, 40, 10, 1, 70], [40] * 6])
+@pytest.mark.parametrize("row", [0, 64, 4096])
+def test_overlapping_qkv_rows(gpu, row, lengths):
+    """qkv rows closer together than they are long, for batches of either side."""
+    announce(test="heads_overlapping_rows", row=row, lengths=lengths)
+    case = prefill_case(gpu, lengths, seed=6)
+    n, width = case["qkv"].shape
+    assert reads_qkv(lengths, 32, row, width) == (lengths == [40] * 6)
+    flat = case["qkv"].reshape(-1)[:(n - 1) * row + width].clone()
+    case["qkv"] = flat.as_strided((n, width), (row, 1))
+    check(case)
+
+
+@pytest.mark.parametrize("lengths", [[33], [130]])
+@pytest.mark.parametrize("row", [33_554_175, 33_554_176, 69_273_700])
+def test_far_apart_qkv_rows(gpu, row, lengths):
+    """As for the gate's rows, on either side."""
+    announce(test="heads_far_qkv_rows", row=row, lengths=lengths)
+    case = prefill_case(gpu, lengths, seed=7)
+    n, width = case["qkv"].shape
+    assert reads_qkv(lengths, 32, row, width) == (row == 33_554_175)
+    far = torch.empty((n - 1) * row + width, dtype=torch.bfloat16, device=gpu)
+    far = far.as_strided((n, width), (row, 1))
+    far.copy_(case["qkv"])
+    case["qkv"] = far
     check(case)

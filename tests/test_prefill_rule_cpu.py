@@ -4,18 +4,31 @@ from __future__ import annotations
 
 import pytest
 
-from tests.prefill_rule import plan, side
+from tests.prefill_rule import plan, reads_qkv, side
 
-LIMIT = (0x7fffffff // 2 - 128) // 31   # largest gate row stride of the whole-head kernels
+LIMIT = (0x7fffffff // 2 - 128) // 32   # largest gate row stride of the whole-head kernels
 
 
 @pytest.mark.parametrize("lengths", [[32], [100] * 8, [300] * 8, [290, 1, 0, 70, 33] + [0] * 254])
 def test_gate_rows_beyond_32_bit_offsets_take_the_norm_pass(lengths):
-    """The last byte of a chunk's gate rows fits 31 bits up to LIMIT; beyond (and for rows that go
+    """A chunk's gate rows and the one after them fit 31 bits up to LIMIT; beyond (and for rows that go
     backwards) no whole-head kernel runs."""
-    assert 2 * (31 * LIMIT + 128) <= 0x7fffffff < 2 * (31 * (LIMIT + 1) + 128)
+    assert 2 * (32 * LIMIT + 128) <= 0x7fffffff < 2 * (32 * (LIMIT + 1) + 128)
     assert plan(lengths, 32, LIMIT) == plan(lengths, 32)
     assert plan(lengths, 32, LIMIT)[1]
     for row in (LIMIT + 1, 70_000_000, 1 << 40, -4096):
         assert plan(lengths, 32, row)[1:] == (False, True)
         assert side(lengths, 32, row) == "rows"
+
+
+@pytest.mark.parametrize("lengths", [[32], [200], [100] * 8, [300] * 8])
+def test_qkv_rows_that_overlap_or_lie_far_apart(lengths):
+    """Overlapping rows (one expanded over the tokens, say) are read by the whole-head kernels
+    alone; rows beyond 31-bit offsets in a chunk, and backward ones, by neither side."""
+    width, rows = 8192, plan(lengths, 32)[2]
+    limit = (0x7fffffff // 2 - width) // 32
+    assert reads_qkv(lengths, 32, width, width) and reads_qkv(lengths, 32, limit, width)
+    for row in (0, 64, width - 1):
+        assert reads_qkv(lengths, 32, row, width) == (not rows)
+    for row in (limit + 1, 1 << 40, -width):
+        assert not reads_qkv(lengths, 32, row, width)
