@@ -430,7 +430,10 @@ __device__ __forceinline__ void prep_head(const PrepTiles& x, const PrepGates& i
     {
       const bool live = token < len;
       const float xa = bf16_to_f32(in.a) + in.dt_bias;
-      const float gl = live ? -__expf(in.a_log) * softplus(xa) : 0.0f;
+      // (a log decay below -1e6, whose decay is 0 in any form, as -1e6: sums in log2 units stay
+      // finite and keep the bits of the decays after it; NaN stays)
+      const float decay = -__expf(in.a_log) * softplus(xa);
+      const float gl = live ? (decay < -1e6f ? -1e6f : decay) : 0.0f;
       const float beta = live ? sigmoid(bf16_to_f32(in.b)) : 0.0f;
       const double sum = prefix_sum32(gl, lane) * 1.4426950408889634;   // exp2 from here on
       const float G = static_cast<float>(sum);

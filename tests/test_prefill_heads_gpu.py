@@ -163,3 +163,19 @@ def test_far_apart_qkv_rows(gpu, row, lengths):
     far.copy_(case["qkv"])
     case["qkv"] = far
     check(case)
+
+
+@pytest.mark.parametrize("lengths", [[5, 33, 64, 1], [270, 290, 300, 280, 265]])
+@pytest.mark.parametrize("value", [3.3e38, float("inf")])
+@pytest.mark.parametrize("where", ["last", "middle"])
+def test_decays_to_zero(gpu, where, value, lengths):
+    """Log decays near -3e38 (finite, but not in units of log 2) and infinite: the state before
+    them is gone, what follows is as from a zero state."""
+    assert side(lengths, 32) == ("own" if len(lengths) == 4 else "records")
+    announce(test="heads_decay_to_zero", where=where, value=value, lengths=lengths)
+    case = prefill_case(gpu, lengths, seed=8)
+    case["a_log"].fill_(-0.1)
+    case["a"] = case["a"].clone()
+    ends = case["cu_seqlens"][1:].long() - 1
+    case["a"][ends if where == "last" else ends - torch.tensor(lengths, device=gpu) // 2] = value
+    check(case)
