@@ -102,14 +102,10 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Where both sides are launched, ahead of chunk_start in the workspace: chunk_start[-1] is the
-// decision (1: whole heads), chunk_start[-16 .. -9] the other scan's queues, one per XCD.
-constexpr int kXcds = 8;
-constexpr int kQueueAt = -15;   // from the decision
-
 // chunk_start[n] = sum over m < n of ceil(L_m / C) for n = 0 .. num_sequences: where the
 // chunks of sequence n begin in the global chunk order.  One workgroup, a block-wide scan per
-// 256 sequences.  With `form` also HeadsRule's decision there, and the scan's queues cleared.
+// 256 sequences.  With `form` (the word ahead of chunk_start, where both sides are launched) also
+// HeadsRule's decision there: 1 for whole heads.
 template <int C>
 __global__ __launch_bounds__(kThreads) void chunk_index_kernel(const int32_t* cu,
                                                                int num_sequences,
@@ -146,7 +142,6 @@ __global__ __launch_bounds__(kThreads) void chunk_index_kernel(const int32_t* cu
     __syncthreads();  // wave_total is rewritten by the next round
   }
   if (form == nullptr) return;
-  if (tid < kXcds) form[kQueueAt + tid] = 0;
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) longest = max(longest, __shfl_xor(longest, d));
   if (lane == 0) wave_longest[wave] = longest;
@@ -686,13 +681,16 @@ __device__ __forceinline__ uint32_t prep32_tile(int index) {
   }
 }
 
+// With `form` (the whole-head kernels' batch if it is set) it returns at once unless that is 0.
 template <bool DtBf16, bool Wide>
-__device__ __forceinline__ void prep32_unit(const DecodeParams& p, int num_sequences, float* ws,
-                                            const int32_t* chunk_start, int records,
-                                            int64_t unit) {   // chunk * H + k-head
+__global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
+void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
+                         const int32_t* chunk_start, int records, const int32_t* form) {
+  if (form != nullptr && *form != 0) return;
   using R = Rec32;
   constexpr int kCs = R::kC;
   constexpr int kTokens = kCs / (kPrep32Threads / 64);   // tokens normalised per wave
+  const int64_t unit = blockIdx.x;   // chunk * H + k-head
   const int g = static_cast<int>(unit / p.num_k_heads);
   if (g >= records) return;
   const int key_head = static_cast<int>(unit - static_cast<int64_t>(g) * p.num_k_heads);
@@ -981,22 +979,6 @@ __device__ __forceinline__ void prep32_unit(const DecodeParams& p, int num_seque
     }
     // the next v-head writes -A after its first barrier (every read of -A and T above is
     // behind one of this v-head's) and its gates went to the other buffer
-  }
-}
-
-// One workgroup per (chunk, k-head), or (Many) a grid that fits the chip and goes over them: with
-// `form` (the whole-head kernels' batch if it is set) a launch in vain then costs 2 us, where
-// 16,384 workgroups that return at once took 8.
-template <bool DtBf16, bool Wide, bool Many>
-__global__ __launch_bounds__(kPrep32Threads) __attribute__((amdgpu_waves_per_eu(5)))
-void chunk_prep32_kernel(const DecodeParams p, int num_sequences, float* ws,
-                         const int32_t* chunk_start, int records, const int32_t* form) {
-  if (form != nullptr && *form != 0) return;
-  const int64_t units = static_cast<int64_t>(records) * p.num_k_heads;
-  for (int64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
-    prep32_unit<DtBf16, Wide>(p, num_sequences, ws, chunk_start, records, unit);
-    if (!Many) return;
-    __syncthreads();   // the LDS tiles are rewritten
   }
 }
 
@@ -1502,14 +1484,17 @@ __device__ __forceinline__ void load_output32(Scan32Output& o, __amdgpu_buffer_r
 // The products with S and with V_new ck on the bf16 matrix cores, each as three products
 // against split4's parts (fp32-exact operands, fp32 sums, 80 VGPRs).  (Prompts of one
 // chunk once kept fp32 products, before the splits took one instruction per remainder.)
-__device__ __forceinline__ void scan32_rows(const DecodeParams& p, int num_sequences, float* ws,
-                                            const int32_t* chunk_start, int records, int xcd,
-                                            int rank) {
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(6)))
+void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
+                         const int32_t* chunk_start, int records, const int32_t* form) {
+  if (form != nullptr && *form != 0) return;   // (the whole-head kernels' batch)
   using R = Rec32;
   constexpr int kCs = R::kC;                 // 32 tokens per chunk
   constexpr int kRows = 32;                  // state rows per workgroup
   constexpr int kBlocks = kDim / kRows;
   // XCD-aware ids as in chunk_scan_kernel: the 4 row blocks of one (sequence, head) on one XCD
+  const int xcd = blockIdx.x & 7;
+  const int rank = blockIdx.x >> 3;
   const int pair = (rank / kBlocks) * 8 + xcd;
   if (pair >= num_sequences * p.num_v_heads) return;
   const int seq = pair / p.num_v_heads;
@@ -1777,32 +1762,6 @@ __device__ __forceinline__ void scan32_rows(const DecodeParams& p, int num_seque
   }
 }
 
-// One workgroup per (pair, row block).  Many: a fixed grid whose workgroups take them from their
-// XCD's queue (see chunk_prep32_kernel; 65,536 workgroups that return at once took 25 us).  The
-// loop's registers cost it two of six waves a SIMD.
-template <bool Many>
-__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(Many ? 4 : 6)))
-void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
-                         const int32_t* chunk_start, int records, int32_t* form) {
-  if (form != nullptr && *form != 0) return;
-  const int xcd = blockIdx.x & (kXcds - 1);
-  int rank = blockIdx.x / kXcds;
-  if constexpr (!Many) {
-    scan32_rows(p, num_sequences, ws, chunk_start, records, xcd, rank);
-  } else {
-    __shared__ int taken;
-    const int ranks = (num_sequences * p.num_v_heads + kXcds - 1) / kXcds * (kDim / 32);
-    while (rank < ranks) {
-      if (threadIdx.x == 0)
-        taken = atomicAdd(form + kQueueAt + xcd, 1) + static_cast<int>(gridDim.x) / kXcds;
-      scan32_rows(p, num_sequences, ws, chunk_start, records, xcd, rank);
-      __syncthreads();   // (and the LDS tiles are rewritten)
-      rank = __builtin_amdgcn_readfirstlane(taken);
-      __syncthreads();
-    }
-  }
-}
-
 template <int C>
 int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
   return num_tokens / C + num_sequences;  // each sequence adds at most one partial chunk
@@ -1818,7 +1777,6 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
 }
 
-constexpr int64_t kManyGroups = 32768;   // of the scan: beyond them the Many kernels
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
                   bool w_bf16, const Plan32& plan, float* ws, int32_t* chunk_start,
@@ -1850,28 +1808,22 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
   }
   // 16-byte pieces of q and k (and v) when every row starts at a 16-byte boundary
   const bool wide = (reinterpret_cast<uintptr_t>(p.qkv) & 15) == 0 && (p.qkv_row & 7) == 0;
-#define LD_PREP(K, ...)                                                                        \
-  (dt_bf16 ? (wide ? K<true, true __VA_ARGS__> : K<true, false __VA_ARGS__>)                   \
-           : (wide ? K<false, true __VA_ARGS__> : K<false, false __VA_ARGS__>))
-#define LD_COMMA ,
+#define LD_PREP(K)                                        \
+  (dt_bf16 ? (wide ? K<true, true> : K<true, false>)      \
+           : (wide ? K<false, true> : K<false, false>))
   if constexpr (TT == 2) {
-    int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
+    const int64_t scan_groups = (pairs + 7) / 8 * 8 * (kDim / 32);
     if (scan_groups > 0x7fffffff) return fail(LD_ERR_INVALID_ARGUMENT, "prefill too large");
-    const bool many = form != nullptr && scan_groups > kManyGroups;
-    const int64_t prep_grid = many ? std::min<int64_t>(prep_groups, 1280) : prep_groups;   // 5 a CU
-    if (many) scan_groups = 1024;
-    const auto prep = many ? LD_PREP(chunk_prep32_kernel, LD_COMMA true)
-                           : LD_PREP(chunk_prep32_kernel, LD_COMMA false);
-    hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_grid)), dim3(kPrep32Threads), 0,
+    const auto prep = LD_PREP(chunk_prep32_kernel);
+    hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kPrep32Threads), 0,
                        stream, p, num_sequences, ws, chunk_start, static_cast<int>(chunks), form);
-    hipLaunchKernelGGL(many ? chunk_scan32_kernel<true> : chunk_scan32_kernel<false>,
-                       dim3(static_cast<uint32_t>(scan_groups)), dim3(kScanThreads), 0, stream, p,
-                       num_sequences, ws, chunk_start, static_cast<int>(chunks), form);
+    hipLaunchKernelGGL(chunk_scan32_kernel, dim3(static_cast<uint32_t>(scan_groups)),
+                       dim3(kScanThreads), 0, stream, p, num_sequences, ws, chunk_start,
+                       static_cast<int>(chunks), form);
   } else {
     const auto prep = LD_PREP(chunk_prep_kernel);
     hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kPrepThreads), 0,
                        stream, p, num_sequences, ws, chunk_start, static_cast<int>(chunks));
-#undef LD_COMMA
 #undef LD_PREP
     // two row tiles per workgroup once they still give 2 workgroups per CU
     const bool two_tiles = pairs * (kDim / 32) >= 512;

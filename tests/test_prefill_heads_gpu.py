@@ -11,7 +11,7 @@ import torch
 from lightdelta_amd import ops
 from oracle.decode import expected_prefill
 from tests.parity import assert_bf16_outputs, assert_states
-from tests.prefill_rule import reads_qkv, side
+from tests.prefill_rule import plan, reads_qkv, side
 from tests.test_prefill_gpu import PREFILL, announce, prefill_case, run
 
 pytestmark = pytest.mark.gpu
@@ -69,8 +69,10 @@ def test_both_sides_of_the_record_rule(gpu, heads, lengths):
 
 @pytest.mark.parametrize("lengths", [[290, 1, 0, 70, 33] + [0] * 254 + [40], [3, 0, 1, 34] * 65])
 def test_many_sequences(gpu, lengths):
-    """Over 8,192 (sequence, head) pairs the row-block scan takes them from queues: a batch for it
-    (one long prompt) and one for the whole-head kernels, each replayed from a graph too."""
+    """Over 8,192 (sequence, head) pairs: a batch for the row-block scan (one long prompt) and one
+    for the whole-head kernels, decided on the device, each replayed from a graph too."""
+    assert all(plan(lengths, 32)[1:])
+    assert side(lengths, 32) == ("rows" if 290 in lengths else "own")
     announce(test="heads_many", sequences=len(lengths))
     case = prefill_case(gpu, lengths, seed=7)
     pool0 = case["pool"].clone()

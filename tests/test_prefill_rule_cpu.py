@@ -32,3 +32,11 @@ def test_qkv_rows_that_overlap_or_lie_far_apart(lengths):
         assert reads_qkv(lengths, 32, row, width) == (not rows)
     for row in (limit + 1, 1 << 40, -width):
         assert not reads_qkv(lengths, 32, row, width)
+
+
+def test_more_pairs_than_the_row_block_grid_holds():
+    """roundup(pairs, 8) x 4 row blocks x 512 threads stays under 2^32; beyond, whole heads alone."""
+    lengths = [40] * 65_534 + [3000]
+    assert (len(lengths) * 32 + 7) // 8 * 8 * 4 * 512 < 1 << 32
+    assert plan(lengths, 32)[1:] == (True, True)
+    assert plan(lengths + [40], 32)[1:] == (True, False)
