@@ -14,6 +14,15 @@ namespace ld {
 // heads' chains the batch keeps going beside its longest: heads x chunks / longest chain, the
 // number of (sequence, head) pairs if the prompts are equally long.  Over short chains the
 // launches and records that the first saves decide.
+//   Where workgroups prepare their own chunks (4.6 us a chunk) the line is 150 such chains.  us,
+// row blocks / whole heads, 32 v-heads: one of 6000 and 300 of 40 tokens (134 chains) 897 / 1020,
+// and 340 (148) 975 / 1040, 20 of 1 to 600 (142) 84 / 96, 22 (149) 97 / 128, one of 512 and 28 of
+// 40 (144) 82 / 100, one of 1024 and 50 of 64 (132) 174 / 189; the other way one of 2048 and 230 of
+// 32 (147) 457 / 430, 24 of 1 to 1500 (130) 226 / 223; beyond, 24 of 1 to 600 (160) 120 / 119, one
+// of 2048 and 250 of 32 (157) 497 / 441, one of 512 and 36 of 40 (176) 98 / 106, 32 of 1 to 1500
+// (171) 303 / 288.  With records (3.3 us) it is 96, about which the order of the prompts decides:
+// 16 of 1 to 3000 (85) 277 / 276, 18 (93) 349 / 293, 11 at 48 v-heads (97) 283 / 257, 5 of 500 to
+// 1500 (115) 187 / 176; 22 of 1 to 8000 (97) 886 / 959, one of 4000 and 8 of 1000 (98) 417 / 466.
 struct HeadsRule {
   int num_v_heads;
   int short_chunks;   // whole heads up to this many chunks in the longest chain
@@ -65,7 +74,7 @@ constexpr Plan32 plan_chunks32(int64_t num_tokens, int64_t num_sequences, int nu
   plan.own = num_tokens <= kOwnTokens * num_sequences;
   plan.rule.num_v_heads = num_v_heads;
   plan.rule.short_chunks = !plan.own ? 0 : pairs > 64 ? 8 : 4;
-  plan.rule.chains = plan.own ? 128 : 96;
+  plan.rule.chains = plan.own ? 150 : 96;
   // (the whole-head kernels' gate offsets are of 32 bits, the norm pass's of 64)
   if (!chunk_rows_fit(gate_row, 128)) {
     plan.rows = true;

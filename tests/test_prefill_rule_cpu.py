@@ -40,3 +40,15 @@ def test_more_pairs_than_the_row_block_grid_holds():
     assert (len(lengths) * 32 + 7) // 8 * 8 * 4 * 512 < 1 << 32
     assert plan(lengths, 32)[1:] == (True, True)
     assert plan(lengths + [40], 32)[1:] == (True, False)
+
+
+@pytest.mark.parametrize("lengths,heads,faster", [
+    ([6000] + [40] * 300, 32, "rows"), ([3000] + [33] * 90, 48, "rows"),
+    ([512] + [40] * 28, 32, "rows"), ([1024] + [64] * 50, 32, "rows"),
+    ([8192] + [20] * 511, 32, "rows"), ([4096] + [16] * 15, 32, "rows"),
+    ([2048] + [32] * 260, 32, "own"), ([512] + [40] * 48, 32, "own"), ([32] * 512, 32, "own"),
+    ([64] * 16, 32, "own"), ([100] * 28 + [2000] * 4, 32, "records"), ([1024] * 32, 32, "records"),
+    ([3000] * 3, 48, "records"), ([1000] * 4, 32, "rows")])
+def test_the_faster_side_is_taken(lengths, heads, faster):
+    """Batches whose two sides were measured 5% or more apart (equal ones of 128 pairs apart)."""
+    assert side(lengths, heads) == faster
