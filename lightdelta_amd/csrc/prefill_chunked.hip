@@ -1481,33 +1481,37 @@ __device__ __forceinline__ void load_output32(Scan32Output& o, __amdgpu_buffer_r
   }
 }
 
+// The lane's number, formed from the count of lanes below it; Fresh: at this very point.
+template <bool Fresh>
+__device__ __forceinline__ int lane_id() {
+  int zero = 0;
+  if constexpr (Fresh) asm volatile("" : "+s"(zero));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 // The products with S and with V_new ck on the bf16 matrix cores, each as three products
 // against split4's parts (fp32-exact operands, fp32 sums, 80 VGPRs).  (Prompts of one
 // chunk once kept fp32 products, before the splits took one instruction per remainder.)
-__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(6)))
-void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
-                         const int32_t* chunk_start, int records, const int32_t* form) {
-  if (form != nullptr && *form != 0) return;   // (the whole-head kernels' batch)
+// Loop: called in a loop, out of which the compiler would move what depends on the lane alone and
+// hold it in registers that the chunk loop needs; so the lane is read anew where noted.
+template <bool Loop>
+__device__ __forceinline__ void scan32_rows(const DecodeParams& p, int num_sequences, float* ws,
+                                            const int32_t* chunk_start, int records, int xcd,
+                                            int rank, int tid) {
   using R = Rec32;
   constexpr int kCs = R::kC;                 // 32 tokens per chunk
   constexpr int kRows = 32;                  // state rows per workgroup
   constexpr int kBlocks = kDim / kRows;
   // XCD-aware ids as in chunk_scan_kernel: the 4 row blocks of one (sequence, head) on one XCD
-  const int xcd = blockIdx.x & 7;
-  const int rank = blockIdx.x >> 3;
   const int pair = (rank / kBlocks) * 8 + xcd;
   if (pair >= num_sequences * p.num_v_heads) return;
   const int seq = pair / p.num_v_heads;
   const int head = pair - seq * p.num_v_heads;
   const int row_block = rank % kBlocks;
   const int row0 = row_block * kRows;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int li = lane & 15;
-  const int lg = lane >> 4;
-  const uint32_t lane16 = static_cast<uint32_t>(lane) * 16;
-  const uint32_t lg16 = static_cast<uint32_t>(lg) * 16;
+  int li, lg;   // lane % 16, lane / 16
+  uint32_t lane16, lg16, voff;
   const int w = wave & 3;
   const int a = w & 1;    // the wave's token tile
   const int h = w >> 1;   // the wave's row tile
@@ -1557,7 +1561,6 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
   };
   // chunk c's rows of qkv (0 bytes past the last chunk, or a sequence's rows past its end:
   // their v reads as zeros), and the lane's offset of v[16 a + 4 lg][row0 + 16 h + li] in it
-  const int v_col = (2 * p.num_k_heads + head) * kDim + row0 + 16 * h + li;
   auto v_rows = [&](int c) {
     const int t0 = bos + min(c, max(chunks - 1, 0)) * kCs;
     return __builtin_amdgcn_make_buffer_rsrc(
@@ -1565,7 +1568,15 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
         c < chunks ? min(kCs, eos - t0) * static_cast<int>(p.qkv_row) * 2 : 0, 0x00020000);
   };
   const uint32_t vrow = static_cast<uint32_t>(p.qkv_row) * 2;
-  const uint32_t voff = (16 * a + 4 * lg) * vrow + static_cast<uint32_t>(v_col) * 2;
+  auto set_lane = [&](int lane) __attribute__((always_inline)) {
+    li = lane & 15;
+    lg = lane >> 4;
+    lane16 = static_cast<uint32_t>(lane) * 16;
+    lg16 = static_cast<uint32_t>(lg) * 16;
+    const int v_col = (2 * p.num_k_heads + head) * kDim + row0 + 16 * h + li;
+    voff = (16 * a + 4 * lg) * vrow + static_cast<uint32_t>(v_col) * 2;
+  };
+  set_lane(tid & 63);
 
   if (wave < 4) {
     // The wave's pieces of the state, S[row0 + 16 hh + li][16 (2w + t) + 4 lg + r], live in
@@ -1623,7 +1634,7 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
     // formed anew from the lane count, mbcnt, as a work-item id or offset held across the
     // chunk loop took a register that loop needs: a spill).
     auto store_own = [&](int t, int hh, f32x4 v) __attribute__((always_inline)) {
-      const int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      const int l = lane_id<Loop>();
       const __amdgpu_buffer_rsrc_t srs = state_resource(p, slot, head, true);
       const uint32_t soff =
           static_cast<uint32_t>(((row0 + (l & 15)) * kDim + 32 * w + 4 * (l >> 4)) * 4);
@@ -1701,6 +1712,7 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
       }
     };
     for (int c = 0; c + 1 < chunks; ++c) chunk(c, std::false_type{});
+    if constexpr (Loop) set_lane(lane_id<Loop>());
     if (chunks > 0) {
       chunk(chunks - 1, std::true_type{});
     } else if (slot > 0) {
@@ -1762,6 +1774,31 @@ void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
   }
 }
 
+// One workgroup per (pair, row block) or, with Loop, per kLoopItems of them, a grid's length apart.
+template <bool Loop>
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(6)))
+void chunk_scan32_kernel(const DecodeParams p, int num_sequences, float* ws,
+                         const int32_t* chunk_start, int records, const int32_t* form) {
+  if (form != nullptr && *form != 0) return;   // (the whole-head kernels' batch)
+  const int xcd = blockIdx.x & 7;
+  int rank = blockIdx.x >> 3;
+  if constexpr (!Loop) {
+    scan32_rows<Loop>(p, num_sequences, ws, chunk_start, records, xcd, rank, threadIdx.x);
+  } else {
+    __shared__ int next;   // (held in a register it would cost the chunk loop one)
+    const int ranks = (num_sequences * p.num_v_heads + 7) / 8 * (kDim / 32);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    while (rank < ranks) {
+      const int tid = 64 * wave + lane_id<true>();
+      if (tid == 0) next = rank + static_cast<int>(gridDim.x >> 3);
+      scan32_rows<Loop>(p, num_sequences, ws, chunk_start, records, xcd, rank, tid);
+      __syncthreads();   // (the LDS tiles are rewritten)
+      rank = __builtin_amdgcn_readfirstlane(next);
+      __syncthreads();
+    }
+  }
+}
+
 template <int C>
 int64_t max_chunks(int64_t num_tokens, int64_t num_sequences) {
   return num_tokens / C + num_sequences;  // each sequence adds at most one partial chunk
@@ -1777,6 +1814,14 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
   return max_chunks<kC>(num_tokens, num_sequences) * num_v_heads * kRecord * 4;
 }
 
+// Over this many of its workgroups the row-block scan is launched a quarter of them, where its
+// launch may be in vain: 65,536 take 18 us to return (us, one workgroup each / loops: 512 x 32
+// 640 / 619, 1024 x 32 1258 / 1213; without the launches 598 and 1180).  Where its batch comes the loops cost or gain: one of 8192 and
+// 511 of 20 tokens 1024 / 1071, the 8192 last 1402 / 1338, one of 4000 and 260 of 20 530 / 560, 260
+// of 17 and one of 3000 627 / 616, one of 14000 and 400 of 20 1200 / 1214.  (Queues on a grid that
+// fits the chip: 1113 and 1770 for the first two, as long chains that share a CU slow each other.)
+constexpr int64_t kLoopGroups = 32768;
+constexpr int kLoopItems = 4;
 template <int TT>
 int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, bool dt_bf16,
                   bool w_bf16, const Plan32& plan, float* ws, int32_t* chunk_start,
@@ -1817,7 +1862,10 @@ int launch_chunks(const DecodeParams& p, int num_sequences, int64_t num_tokens, 
     const auto prep = LD_PREP(chunk_prep32_kernel);
     hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(prep_groups)), dim3(kPrep32Threads), 0,
                        stream, p, num_sequences, ws, chunk_start, static_cast<int>(chunks), form);
-    hipLaunchKernelGGL(chunk_scan32_kernel, dim3(static_cast<uint32_t>(scan_groups)),
+    const bool loop = form != nullptr && scan_groups > kLoopGroups;
+    const int64_t scan_grid = loop ? (scan_groups / 8 + kLoopItems - 1) / kLoopItems * 8 : scan_groups;
+    hipLaunchKernelGGL(loop ? chunk_scan32_kernel<true> : chunk_scan32_kernel<false>,
+                       dim3(static_cast<uint32_t>(scan_grid)),
                        dim3(kScanThreads), 0, stream, p, num_sequences, ws, chunk_start,
                        static_cast<int>(chunks), form);
   } else {

@@ -58,15 +58,10 @@ struct Plan32 {
 constexpr int64_t kRowPairs = (1 << 21) - 8;
 
 // Where the host's numbers leave no choice only one side is launched; else both are, and the
-// other side's workgroups return at once: 4 to 10 us of launches, 20 to 40 where whole heads run
-// over 8,192 pairs and more (65,536 row-block workgroups take 18 us to return; us, one side / both:
-// 512 x 32 620 / 640, 1024 x 32 1216 / 1257).  A grid that fits the chip and takes its workgroups'
-// pairs from a queue returns in 2 us but is slower where its batch comes: one of 8192 and 511 of
-// 20 tokens 1,203 us against 1,028 (1,020 by the row blocks alone), with the 8192 last 1,619
-// against 1,404; at six waves a SIMD and without spills still 1,113 and 1,770.  us, row blocks /
-// whole heads / decided: 32 x 1024 985 / 586 / 590, 512 prompts of 8 to 56 994 / 631 / 680, 16 x 64
-// 52 / 32 / 40, one of 4096 and 15 of 16 277 / 430 / 284, one of 1000 and 30 of 40 108 / 162 / 112,
-// 5 of 1 to 6000 179 / 272 / 184, 32 of 1 to 1000 206 / 179 / 191.
+// other side's workgroups return at once: 4 to 10 us of launches (us, row blocks / whole heads / so
+// decided: 32 x 1024 985 / 586 / 590, 512 prompts of 8 to 56 994 / 631 / 660, 16 x 64 52 / 32 / 40,
+// one of 4096 and 15 of 16 277 / 430 / 284, one of 1000 and 30 of 40 108 / 162 / 112, 5 of 1 to 6000
+// 179 / 272 / 184, 32 of 1 to 1000 206 / 179 / 191).
 constexpr Plan32 plan_chunks32(int64_t num_tokens, int64_t num_sequences, int num_v_heads,
                                int64_t gate_row) {
   const int64_t pairs = num_sequences * num_v_heads;

@@ -67,12 +67,14 @@ def test_both_sides_of_the_record_rule(gpu, heads, lengths):
     check(prefill_case(gpu, lengths, heads=heads, seed=sum(lengths), dt_dtype=torch.bfloat16))
 
 
-@pytest.mark.parametrize("lengths", [[290, 1, 0, 70, 33] + [0] * 254 + [40], [3, 0, 1, 34] * 65])
+@pytest.mark.parametrize("lengths", [[290, 1, 0, 70, 33] + [0] * 254 + [40], [3, 0, 1, 34] * 65,
+                                     [33] + [0] * 255 + [300, 7, 0]])
 def test_many_sequences(gpu, lengths):
-    """Over 8,192 (sequence, head) pairs: a batch for the row-block scan (one long prompt) and one
-    for the whole-head kernels, decided on the device, each replayed from a graph too."""
+    """Over 8,192 (sequence, head) pairs: batches for the row-block scan (one long prompt, its
+    workgroups' first or last item) and one for the whole-head kernels, decided on the device,
+    each replayed from a graph too."""
     assert all(plan(lengths, 32)[1:])
-    assert side(lengths, 32) == ("rows" if 290 in lengths else "own")
+    assert side(lengths, 32) == ("rows" if max(lengths) > 256 else "own")
     announce(test="heads_many", sequences=len(lengths))
     case = prefill_case(gpu, lengths, seed=7)
     pool0 = case["pool"].clone()
