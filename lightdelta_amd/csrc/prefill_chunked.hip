@@ -1816,10 +1816,11 @@ int64_t records_bytes(int64_t num_tokens, int64_t num_sequences, int64_t num_v_h
 
 // Over this many of its workgroups the row-block scan is launched a quarter of them, where its
 // launch may be in vain: 65,536 take 18 us to return (us, one workgroup each / loops: 512 x 32
-// 640 / 619, 1024 x 32 1258 / 1213; without the launches 598 and 1180).  Where its batch comes the loops cost or gain: one of 8192 and
-// 511 of 20 tokens 1024 / 1071, the 8192 last 1402 / 1338, one of 4000 and 260 of 20 530 / 560, 260
-// of 17 and one of 3000 627 / 616, one of 14000 and 400 of 20 1200 / 1214.  (Queues on a grid that
-// fits the chip: 1113 and 1770 for the first two, as long chains that share a CU slow each other.)
+// 640 / 619, 1024 x 32 1258 / 1213).  Where its batch comes the loops cost or gain: one of 8192
+// and 511 of 20 tokens 1023 / 1071, the 8192 last 1400 / 1338, one of 4000 and 260 of 20 530 / 560,
+// 260 of 17 and one of 3000 628 / 617, one of 14000 and 400 of 20 1200 / 1213.  (Queues on a grid
+// that fits the chip: 1113 and 1770 for the first two, as long chains that share a CU slow each
+// other.)
 constexpr int64_t kLoopGroups = 32768;
 constexpr int kLoopItems = 4;
 template <int TT>

@@ -35,11 +35,13 @@ def check(case):
     assert torch.equal(case["pool"][0], before[0])
 
 
-@pytest.mark.parametrize("heads", [(1, 1), (2, 6), (16, 16), (4, 32), (16, 48)])
-def test_chunk_edges(gpu, heads):
-    """Lengths one below, at and above one, two and three chunks, one token, none; zero and
-    given initial states; a padding slot."""
-    lengths = [1, 31, 32, 33, 0, 63, 64, 65, 96, 97, 2]
+@pytest.mark.parametrize("heads,times", [((1, 1), 12), ((2, 6), 2), ((16, 16), 1), ((4, 32), 1),
+                                         ((16, 48), 1)])
+def test_chunk_edges(gpu, heads, times):
+    """Lengths one below, at and above one, two and three chunks, one token, none (repeated until
+    there are sequences enough for whole heads); zero and given initial states; a padding slot."""
+    lengths = [1, 31, 32, 33, 0, 63, 64, 65, 96, 97, 2] * times
+    assert side(lengths, heads[1]) == "own"
     announce(test="heads_chunk_edges", heads=heads, lengths=lengths)
     case = prefill_case(gpu, lengths, heads=heads, seed=heads[1], dt_dtype=torch.bfloat16,
                         w_dtype=torch.bfloat16)
@@ -48,21 +50,39 @@ def test_chunk_edges(gpu, heads):
     check(case)
 
 
-@pytest.mark.parametrize("lengths", [[128], [129], [128, 128], [129, 128], [256] * 4,
-                                     [257, 256, 256, 256], [80, 33, 70, 81, 90],
-                                     [330, 40, 10, 1, 70], [300, 256, 280, 270, 256]])
-def test_both_sides_of_the_rule(gpu, lengths):
+@pytest.mark.parametrize("heads,times", [((1, 1), 24), ((2, 6), 4), ((16, 16), 2), ((4, 32), 1),
+                                         ((16, 48), 1)])
+def test_record_chunk_edges(gpu, heads, times):
+    """The same where the chunks' records come from a launch ahead."""
+    lengths = [257, 288, 289, 319, 321, 290, 0, 577] * times
+    assert side(lengths, heads[1]) == "records"
+    announce(test="heads_record_chunk_edges", heads=heads, lengths=lengths)
+    case = prefill_case(gpu, lengths, heads=heads, seed=heads[1], w_dtype=torch.bfloat16)
+    case["has_initial"][1::2] = False
+    case["slots"][3] = -1
+    check(case)
+
+
+@pytest.mark.parametrize("lengths,taken", [
+    ([128], "own"), ([129], "rows"), ([64, 64], "own"), ([128, 128], "rows"), ([129, 128], "rows"),
+    ([86, 85, 85], "own"), ([86, 85, 86], "rows"), ([64] * 4, "own"), ([65, 64, 64, 64], "rows"),
+    ([256] * 4, "rows"), ([257, 256, 256, 256], "rows"), ([80, 33, 70, 81, 90], "own"),
+    ([330, 40, 10, 1, 70], "rows"), ([300, 256, 280, 270, 256], "records")])
+def test_both_sides_of_the_rule(gpu, lengths, taken):
     """Batches of up to 128 (sequence, head) pairs at the limits of the short chains, and 160 pairs,
     decided on the device: short prompts, a long one among short ones, equal longer ones."""
-    announce(test="heads_rule", lengths=lengths)
+    assert side(lengths, 32) == taken
+    announce(test="heads_rule", lengths=lengths, taken=taken)
     check(prefill_case(gpu, lengths, seed=len(lengths)))
 
 
-@pytest.mark.parametrize("heads,lengths", [((16, 48), [290, 353, 261]), ((16, 48), [256] * 3),
-                                           ((16, 32), [270, 250, 250, 250, 250])])
-def test_both_sides_of_the_record_rule(gpu, heads, lengths):
+@pytest.mark.parametrize("heads,lengths,taken", [
+    ((16, 48), [290, 353, 261], "records"), ((16, 48), [256] * 3, "own"),
+    ((16, 32), [270] + [250] * 5, "own"), ((16, 32), [270, 253, 253, 253, 252], "records")])
+def test_both_sides_of_the_record_rule(gpu, heads, lengths, taken):
     """A mean of up to 256 tokens, where a workgroup prepares its chunks itself (nine of them
     here: three rounds of four), and above, where a launch ahead writes their records."""
+    assert side(lengths, heads[1]) == taken
     announce(test="heads_records", heads=heads, lengths=lengths)
     check(prefill_case(gpu, lengths, heads=heads, seed=sum(lengths), dt_dtype=torch.bfloat16))
 
@@ -94,6 +114,7 @@ def test_many_sequences(gpu, lengths):
 @pytest.mark.parametrize("lengths", [[70, 33, 1, 0, 64, 90], [300, 270, 0, 290, 280, 500]])
 @pytest.mark.parametrize("what", ["qkv", "gate", "out"])
 def test_unaligned_rows_give_the_aligned_bits(gpu, what, lengths):
+    assert side(lengths, 32) == ("own" if 33 in lengths else "records")
     announce(test="heads_unaligned", what=what, lengths=lengths)
     case = prefill_case(gpu, lengths, seed=3)
     pool0 = case["pool"].clone()
@@ -118,6 +139,7 @@ def test_unaligned_rows_give_the_aligned_bits(gpu, what, lengths):
 
 def test_rows_of_one_shared_token(gpu):
     """qkv and gate as one row expanded over the tokens (row stride 0)."""
+    assert side([40] * 6, 32, 0) == "own"
     announce(test="heads_expanded_rows")
     case = prefill_case(gpu, [40] * 6, seed=4)
     n = case["qkv"].shape[0]
