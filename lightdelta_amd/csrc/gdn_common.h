@@ -114,20 +114,22 @@ __device__ __forceinline__ float softplus(float x) {
   return y < 1e-4f ? y * (1.0f - 0.5f * y) : __logf(1.0f + y);
 }
 
-// Chunked prefill (prefill_chunked.hip): workspace bytes for num_tokens rows in
-// num_sequences sequences and num_v_heads heads, and the launch of its three phases; the
-// raw outputs go to p.out for prefill_norm_kernel.
 // The form AUTO runs, from the mean prompt length L = num_tokens / num_sequences, measured
-// on MI355X over 1 x 8 .. 4096 x 8 tokens at 32 v heads (ms, token-serial / 64-token
-// chunks / 32-token chunks):
-//   * token-serial below 17 tokens (1024 x 12: 1.30 / - / 1.51; 1024 x 16: 1.53-1.78 /
-//     3.03 / 1.50-1.55; 1 x 16: 0.026 / 0.032 / 0.030);
+// on MI355X at 32 v heads from given states (us, token-serial / 64-token chunks / 32-token
+// chunks):
+//   * token-serial below 17 tokens.  The line is the row-block scan's (1024 x 12: 1300 / - / 1510
+//     by it).  By whole heads, which these batches run, the 32-token form is even from 12 to 13
+//     tokens on (1024 x 10: 1033 / - / 1063; x 12: 1184 / 3000 / 1072; x 16: 1391 / 3010 / 1103;
+//     200 x 12: 238 / - / 240; x 16: 290 / - / 244; 64 x 12: 83 / - / 84; x 16: 100 / - / 85), and
+//     few prompts are within 2 us (1 x 16: 22 / 31 / 20; 16 x 8: 25 / - / 26; 16 x 16: 37 / - /
+//     25): moving it would gain 10 to 25% at 13 to 16 tokens, and change what
+//     ld_gdn_prefill_auto_chunked promises;
 //   * 64-token chunks for prompts of 512 tokens or more in fewer than 64 (sequence, head)
 //     pairs, where the chunk-by-chunk chain is the time and 64-token chunks halve it
-//     (1 x 4096: 2.74 / 0.201 / 0.279; 1 x 512: 0.357 / 0.051 / 0.056; 1 x 256: 0.183 /
-//     0.043 / 0.038; 2 x 2048, 64 pairs: 1.38 / 0.199 / 0.167);
-//   * 32-token chunks otherwise (1024 x 17: 1.63 / 3.06 / 1.53; 1024 x 32: 2.66 / 3.12 /
-//     1.20; 32 x 1024: 2.66 / 1.36 / 0.59; 1 x 64: 0.053 / 0.033 / 0.020).
+//     (1 x 4096: 2735 / 214 / 275; 1 x 512: 350 / 48 / 53; 1 x 256: 179 / 41 / 36; 2 x 2048, 64
+//     pairs: 1390 / 208 / 168);
+//   * 32-token chunks otherwise (1024 x 17: 1505 / 3029 / 1118; 1024 x 32: 2501 / 3137 / 1248;
+//     32 x 1024: 2624 / 1314 / 592; 1 x 64: 51 / 32 / 20).
 // Returns the tokens per chunk (64 or 32), or 0 for the token-serial form.
 inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
                                      int64_t num_v_heads) {
@@ -138,15 +140,17 @@ inline int prefill_auto_chunk_tokens(int64_t num_tokens, int64_t num_sequences,
   return 32;
 }
 
+// Chunked prefill (prefill_chunked.hip): workspace bytes for num_tokens rows in num_sequences
+// sequences and num_v_heads heads.
 int64_t prefill_chunked_workspace_bytes(int64_t num_tokens, int64_t num_sequences,
                                         int64_t num_v_heads);
-// chunk_tokens: 64 or 32
 // What a chunked prefill leaves in `out`: the final outputs (normed), or the raw ones unless
 // *form is set (null: raw).
 struct ChunkedOut {
   bool normed = false;
   const int32_t* form = nullptr;
 };
+// Its launches.  chunk_tokens: 64, or 32 (whose side or sides prefill_rule.h gives).
 int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num_tokens,
                            bool dt_bf16, bool w_bf16, int chunk_tokens, void* workspace,
                            hipStream_t stream, ChunkedOut* result);
@@ -156,7 +160,6 @@ int launch_prefill_chunked(const DecodeParams& p, int num_sequences, int64_t num
 constexpr int64_t kHeadRecordBytes = 9728;
 int launch_chunk_heads(const DecodeParams& p, int num_sequences, bool own, float* ws,
                        const int32_t* chunk_start, const int32_t* form, int records,
-                       bool dt_bf16, bool w_bf16,
-                       hipStream_t stream);
+                       bool dt_bf16, bool w_bf16, hipStream_t stream);
 
 }  // namespace ld

@@ -16,8 +16,7 @@
 // Per chunk and wave (rows past the sequence's end are zeros):
 //   Y = K S^T, O = Q S^T    (q, k as stored against S's exact three-way split: 24 products each)
 //   X = V - diag(ws) Y
-//   V_new = T X             (T = (I + A)^-1 diag(beta); six products of planes: all but those
-//                           below 2^-26 of |T| |X|)
+//   V_new = T X             (T = (I + A)^-1 diag(beta); six of the nine products of planes)
 //   O = diag(sq) O + P X    (P = P0 T: P0 V_new without waiting for V_new; the same)
 //   S' = exp(G_n-1) S + K^T (ck V_new)   (24 products)
 // and the chunk's raw outputs go through LDS (bf16, the reference's rounding point) to the
@@ -25,17 +24,25 @@
 // by ds_read_b64_tr_b16; T, P (as planes) and the per-token scales are prepared by the
 // workgroup itself (short prompts) or come as records from a launch ahead.
 //
-// What bounds it: vector issue and power.  A wave's chunk is 96 matrix instructions (3,072
-// cycles) and, with the norm, 880 vector ones (3,900 cycles of issue with the matrix ones');
-// two workgroups a CU take 8,700 cycles for a chunk each.  At 32 x 1024 tokens and 32 v-heads
-// that is 0.94 PFLOP/s of bf16 products, at a clock that the card's power limit holds at 1.6
-// GHz (a large bf16 GEMM reaches 1.17), 438 us, where chunk_scan32_kernel and the norm pass
-// took 820 us: with a head's rows over four workgroups every wave re-read S's planes from LDS
-// and the raw outputs crossed HBM twice more.  The whole prefill, with the prep
-// below, went from 985 to 585 us there, 257 to 169 us at 8 x 1024, 1,710 to 1,195 us at
-// 1024 x 32.  Products and vector work
-// are laid out by hand, slot by slot: as the compiler scheduled the same code, 32 x 1024 took
-// 685 us.
+// Of the planes' products of T X and P X, those of planes (1, 2), (2, 1) and (2, 2) are left out.
+// A plane 1 is up to 2^-8 and a plane 2 up to 2^-17 of its value, so a term t x lacks up to 2^-24
+// of |t x| (two products of up to 2^-25): the size of an fp32 rounding, one of which each term of
+// the fp32 products that the row-block scan forms here has.  The states' relative error against
+// 64 bits is 0.9e-7 to 1.0e-7, the row blocks' 1.9e-7 to 7.3e-7 (for the decays' sums, below).
+//
+// What bounds it: vector issue, and matrix instructions beside it.  A wave's chunk is 96 matrix
+// instructions (3,072 cycles of a matrix core) and, with the norm and its share of the rest, 900
+// vector ones (4,100 cycles of issue with the matrix ones').  With two workgroups a CU a chunk
+// takes 10,800 cycles, of which a SIMD's vector issue is busy 8,300 and its matrix core 6,100
+// (counters at 32 x 1024 tokens and 32 v-heads, 433 us at 1.89 GHz; 2.33 GHz where fewer
+// workgroups run, so the power limit has a part).  That is 0.95 PFLOP/s of bf16 products (a large
+// bf16 GEMM reaches 1.17), where chunk_scan32_kernel and the norm pass took 820 us: with a head's
+// rows over four workgroups every wave re-read S's planes from LDS and the raw outputs crossed
+// HBM twice more.  The whole prefill, with the prep below, went from 992 to 576 us there, 257 to
+// 169 us at 8 x 1024, 1,710 to 1,213 us at 1024 x 32.  Products and vector work are laid out by
+// hand, slot by slot: as the compiler scheduled the same code, 32 x 1024 took 685 us.  Spilled
+// registers: none with records ahead, 15 where the workgroups prepare their chunks (17 and 47
+// where rows are not at 16-byte boundaries).
 #include "chunk_common.h"
 
 namespace ld {

@@ -36,7 +36,9 @@ struct HeadsRule {
 // saves the record launch and the records (us, with records / own: 1 x 64 26.5 / 19.7, 16 x 64
 // 41.9 / 31.9, 8 x 128 39.5 / 28.4, 8 x 256 53.2 / 49.4, 32 x 256 169 / 155, 1024 x 32 1266 /
 // 1196) but lengthens a chunk's step in its chain by 1 us (13 prompts up to 3000 tokens 265 / 338,
-// 8 x 1024 161 / 177).
+// 8 x 1024 161 / 177).  With the chip full the other workgroup of a CU covers that, and the rule,
+// which looks at the mean alone, gives up 1 to 3% beyond it: 32 x 1024 610 / 591, 64 x 512 607 / 589,
+// 32 x 2048 1141 / 1118, 64 x 300 405 / 395, 16 x 1024 306 / 298, 13 x 1000 268 / 271.
 constexpr int64_t kOwnTokens = 256;
 
 // Whether a chunk's 32 rows (`used` elements of 2 bytes, `row` elements apart), and the row

@@ -31,7 +31,9 @@ constexpr int kPrefillGroup = 4;
 // State tiles that the Infinity Cache (256 MB) holds.  Up to them plain loads and stores are the
 // faster where a call meets the states it left there (us, plain / non-temporal system-scope, 32
 // v-heads: 64 x 3 tokens 46 / 52, 96 x 3 67 / 77, 128 x 3 97 / 101); beyond, the others (160 x 3
-// 130 / 126, 200 x 3 177 / 155, 200 x 1..20 206 / 193, 1024 x 8 909 / 835).
+// 130 / 126, 200 x 3 177 / 155, 200 x 1..20 206 / 193, 1024 x 8 909 / 835; over four pools in turn,
+// so that no call meets its states in a cache, 128 x 3 120 / 120, 160 x 3 146 / 127, 200 x 3 179 /
+// 158, 200 x 1..20 231 / 217, 1024 x 8 over three 914 / 867).
 constexpr int64_t kCachedTiles = 4096;
 
 // One workgroup per (sequence, v-head), wave w holding rows 32w .. 32w + 31.  Tokens go in
