@@ -60,8 +60,9 @@ struct Plan32 {
 constexpr int64_t kRowPairs = (1 << 21) - 8;
 
 // Where the host's numbers leave no choice only one side is launched; else both are, and the
-// other side's workgroups return at once: 4 to 10 us of launches (us, row blocks / whole heads / so
-// decided: 32 x 1024 985 / 586 / 590, 512 prompts of 8 to 56 994 / 631 / 660, 16 x 64 52 / 32 / 40,
+// other side's workgroups return at once: 4 to 10 us of launches, 20 over 8,192 pairs (us, row blocks
+// / whole heads / so
+// decided: 32 x 1024 985 / 586 / 590, 512 prompts of 8 to 56 994 / 631 / 658, 16 x 64 52 / 32 / 40,
 // one of 4096 and 15 of 16 277 / 430 / 284, one of 1000 and 30 of 40 108 / 162 / 112, 5 of 1 to 6000
 // 179 / 272 / 184, 32 of 1 to 1000 206 / 179 / 191).
 constexpr Plan32 plan_chunks32(int64_t num_tokens, int64_t num_sequences, int num_v_heads,
